@@ -767,22 +767,24 @@ S2Args s2_args(gempic_splitting2d *h, double dt, int op)
     // a SIMD issues from its oldest wave first: with equal chunks the later
     // waves of each SIMD run the end of the pass with the SIMD to themselves.
     // Wave w is generation g = w / 4 on its SIMD; chunks weighted 1 + skew
-    // (G - 1 - 2g) / (G - 1) let the generations end together (the
-    // workgroup's total stays kw * chunk).
+    // (G - 1 - 2g) / (G - 1) let the generations end together. Wave w ends
+    // where the running sum of the weights (kw in all) times the waves of 64
+    // particles per wave rounds to, so the chunks tile the workgroup's
+    // kw * chunk particles exactly at every count (rounding each chunk by
+    // itself overran them, e.g. 2 * 1.25 and 2 * 0.75 both up).
     const int G = kw / 4;
     const int64_t per = a.chunk / kWave;              // waves of 64 particles per wave
+    const double skew = G >= 2 ? kS2GenSkew : 0.0;
+    double wsum = 0.0;
     int64_t acc = 0;
     for (int w = 0; w < kw; ++w) {
-        int64_t c = per;
-        if (G >= 2 && kS2GenSkew > 0.0) {
-            const int g = w / 4;
-            const double wt = 1.0 + kS2GenSkew * (double)(G - 1 - 2 * g) / (double)(G - 1);
-            c = w + 1 < kw ? std::max<int64_t>(0, std::llround((double)per * wt)) : per * kw - acc;
-            if (c < 0) c = 0;
-        }
+        if (G >= 2) wsum += 1.0 + skew * (double)(G - 1 - 2 * (w / 4)) / (double)(G - 1);
+        else wsum += 1.0;
+        int64_t end = w + 1 < kw ? std::llround((double)per * wsum) : per * kw;
+        end = std::min<int64_t>(std::max<int64_t>(end, acc), per * kw);
         a.woff[w] = acc * kWave;
-        a.wch[w] = c * kWave;
-        acc += c;
+        a.wch[w] = (end - acc) * kWave;
+        acc = end;
     }
     return a;
 }

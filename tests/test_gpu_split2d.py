@@ -152,6 +152,23 @@ def test_gpu_2d3v_landau_4m_substeps_match_oracle():
             _close(h.b_dofs[c], o_b[c], REL, f"{name} B{c + 1}")
 
 
+@pytest.mark.parametrize("n", [200001, 300001, 1400001])
+def test_gpu_2d3v_every_particle_once(n):
+    """Counts whose weighted wave chunks round up (2 and 6 waves of particles
+    per wave): each particle is pushed and deposited exactly once."""
+    print(f"2d3v wave chunks: n={n}", flush=True)
+    w = _hot(n=n, seed=6)
+    h, pg, osp, o_parts, o_e, o_b = _pair(w, 3, sync=False)
+    h.strang_splitting(0.1, 1)
+    osp.strang_splitting(0.1, 1)
+    h.to_host()
+    for r in range(5):
+        _close(pg.array[r], o_parts[r], 1e-11, f"row {r}")
+    for c in range(3):
+        _close(h.e_dofs[c], o_e[c], 1e-11, f"E{c + 1}")
+        _close(h.b_dofs[c], o_b[c], 1e-11, f"B{c + 1}")
+
+
 def test_gpu_2d3v_errors_and_order():
     w = _hot(n=1000)
     h, pg, *_ = _pair(w, 3)
