@@ -299,13 +299,31 @@ __device__ __forceinline__ double gather(const double (&b)[P + 1], const double 
 constexpr int kPad = 4;
 
 
-__device__ __forceinline__ void load_padded(double *dst, const double *src, int nx)
+// The NF fields src(0), src(1), ... staged one behind the other at dst, each
+// nx + 2 kPad doubles, two loads of a thread in flight: one round trip to
+// memory for all of them (up to 512 doubles), where a copy per field waited
+// for each in turn (a workgroup's start took 6200 cycles, FIXME now).
+template <int NF, class Src>
+__device__ __forceinline__ void stage_padded(double *dst, int nx, Src src)
 {
-    for (int i = threadIdx.x; i < nx + 2 * kPad; i += blockDim.x) {
-        int k = i - kPad;
+    const int nxp = nx + 2 * kPad, tot = NF * nxp;
+    auto value = [&](int i) {
+        int f = 0, k = i - kPad;
+#pragma unroll
+        for (int g = 1; g < NF; ++g)
+            if (i >= g * nxp) {
+                f = g;
+                k = i - g * nxp - kPad;
+            }
         while (k < 0) k += nx;
         while (k >= nx) k -= nx;
-        dst[i] = src[k];
+        return src(f)[k];
+    };
+    for (int i = threadIdx.x; i < tot; i += 2 * kBlock) {
+        const int i2 = i + kBlock;
+        const double a = value(i), b = value(i2 < tot ? i2 : i);
+        dst[i] = a;
+        if (i2 < tot) dst[i2] = b;
     }
 }
 
@@ -522,10 +540,11 @@ __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *
     if (iters > 0) load_particle(tid, nx_x, nx_v1, nx_v2, nx_w);
     if (kPrefetch > 1 && iters > 1) load_particle(tid + kBlock, n2_x, n2_v1, n2_v2, n2_w);
 
-    load_padded(pE1, a.grid + S_E1 * nx, nx);
-    load_padded(pE2p, a.grid + S_E2P * nx, nx);
-    load_padded(pE2, a.grid + S_E2 * nx, nx);
-    load_padded(pB, a.grid + S_B * nx, nx);
+    // E1 alone in 1d1v, none for the charge deposit
+    if constexpr (!RHO_ONLY)
+        stage_padded<V1 ? 1 : 4>(pE1, nx, [&](int f) {
+            return a.grid + (f == 0 ? S_E1 : f == 1 ? S_E2P : f == 2 ? S_E2 : S_B) * nx;
+        });
     for (int i = tid; i < kWaves * NDEP * nx; i += kBlock) rows[i] = 0.0;
     __syncthreads();
     double *myrow = rows + wave * NDEP * nx;
@@ -783,7 +802,8 @@ __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *
         __syncthreads();
         const int len = NDEP * nx;
         for (int idx = tid; idx < len; idx += kBlock) {
-            if (!((DEPMASK >> (idx / nx)) & 1u)) continue;
+            const int r = (idx >= nx) + (idx >= 2 * nx) + (idx >= 3 * nx);
+            if (!((DEPMASK >> r) & 1u)) continue;
             double s = 0.0;
             for (int wv = 0; wv < kWaves; ++wv) s += rows[wv * len + idx];
             a.part[(size_t)bid * len + idx] = s;
@@ -1576,9 +1596,9 @@ __global__ void __launch_bounds__(kBlock) k_boris1d(PassArgs a)
     double *slots = rows + kWaves * NDEP * nx + wave * (kSlotsPerLane * kWave);
     const double *sE1 = pE1 + kPad, *sE2 = pE2 + kPad, *sB = pB + kPad;
     if constexpr (KICK) {
-        load_padded(pE1, a.grid + S_E1M * nx, nx);
-        load_padded(pE2, a.grid + S_E2M * nx, nx);
-        load_padded(pB, a.grid + S_BM * nx, nx);
+        stage_padded<3>(pE1, nx, [&](int f) {
+            return a.grid + (f == 0 ? S_E1M : f == 1 ? S_E2M : S_BM) * nx;
+        });
     }
     for (int i = tid; i < kWaves * NDEP * nx; i += kBlock) rows[i] = 0.0;
     __syncthreads();
@@ -1701,7 +1721,8 @@ __global__ void __launch_bounds__(kBlock) k_boris1d(PassArgs a)
         constexpr unsigned MASK = (1u << D_J1) | (1u << D_J2A);
         const int len = NDEP * nx;
         for (int idx = tid; idx < len; idx += kBlock) {
-            if (!((MASK >> (idx / nx)) & 1u)) continue;
+            const int r = (idx >= nx) + (idx >= 2 * nx) + (idx >= 3 * nx);
+            if (!((MASK >> r) & 1u)) continue;
             double t = 0.0;
             for (int wv = 0; wv < kWaves; ++wv) t += rows[wv * len + idx];
             a.part[(size_t)blockIdx.x * len + idx] = t;
@@ -2659,18 +2680,13 @@ __device__ __forceinline__ void adj1d_body(const AdjArgs &A, int bid, double *sm
     const double *sE1 = pE1 + kPad, *sE2 = pE2 + kPad, *sB = pB + kPad, *sE2p = pE2p + kPad;
     const double *sM1 = pM1 + kPad, *sM2 = pM2 + kPad;
 
-    if constexpr (!POIS) {
-        const double *F = A.fields;
-        load_padded(pE1, F + H_E1 * nx, nx);
-        load_padded(pE2, F + H_E2 * nx, nx);
-        load_padded(pB, F + H_B * nx, nx);
-        load_padded(pE2p, F + H_E2P * nx, nx);
-    }
-    if constexpr (REV) {
-        load_padded(pM1, A.agrid + A_MU1 * nx, nx);
-        load_padded(pM2, A.agrid + A_MU2 * nx, nx);
-    }
-    if constexpr (POIS) load_padded(pM1, A.agrid + A_NU * nx, nx);
+    if constexpr (POIS)
+        stage_padded<1>(pM1, nx, [&](int) { return A.agrid + A_NU * nx; });
+    else
+        stage_padded<REV ? 6 : 4>(pE1, nx, [&](int f) {
+            const double *F = A.fields + (f == 0 ? H_E1 : f == 1 ? H_E2 : f == 2 ? H_B : H_E2P) * nx;
+            return f < 4 ? F : A.agrid + (f == 4 ? A_MU1 : A_MU2) * nx;
+        });
     for (int i = tid; i < kWaves * NDEP * nx; i += kBlock) rows[i] = 0.0;
     __syncthreads();
     double *myrow = rows + wave * NDEP * nx;
@@ -3019,7 +3035,8 @@ __device__ __forceinline__ void adj1d_body(const AdjArgs &A, int bid, double *sm
                                   (1u << AR_SCAL);
         const int len = NDEP * nx;
         for (int idx = tid; idx < len; idx += kBlock) {
-            if (!((MASK >> (idx / nx)) & 1u)) continue;
+            const int r = (idx >= nx) + (idx >= 2 * nx) + (idx >= 3 * nx);
+            if (!((MASK >> r) & 1u)) continue;
             double s = 0.0;
             for (int wv = 0; wv < kWaves; ++wv) s += rows[wv * len + idx];
             a.part[(size_t)bid * len + idx] = s;
