@@ -85,10 +85,28 @@ struct Launch {
     int ngroups;
 };
 
+// Workgroups of a 1D particle pass: 4 particles per thread, fewer (down to
+// one) while that makes under 512 workgroups, two per CU. A workgroup's start
+// and drain cost about 8 us against 0.5 us per particle of a lane, so a small
+// count wants the chip filled first. us per step at (least particles per
+// thread, workgroups below which it does not apply) = (8, 0), (8, 256),
+// (4, 256), (4, 512):
+//   fused 1D2V     16,384: 35.7, 19.2, 19.3, 19.2   300,001: 34.4, 31.5, 31.7, 31.1
+//               1,048,576: 41.3, 41.7, 33.2, 33.4
+//   1D1V (hot)    100,000: 46.1, 24.2, 24.3, 22.0   400,000: 40.8, 38.2, 33.2, 33.2
+//   24 instances of 65,536 to 524,288 particles in one ensemble, whose
+//   workgroups fill the chip together: 164, 175, 176, 181
+// An ensemble's instances keep their stand-alone partition (equal results),
+// so it pays for the small counts' gain; gempic_ensemble_autotune sets larger
+// chunks.
+constexpr int kPerThread = 4;
+constexpr int kFewBlocks = 512;
+
 Launch plan(int64_t n, int max_blocks)
 {
     Launch L;
-    int64_t want = (n + (int64_t)kBlock * 8 - 1) / ((int64_t)kBlock * 8);   // >= 8 particles per thread
+    int64_t want = (n + (int64_t)kBlock * kPerThread - 1) / ((int64_t)kBlock * kPerThread);
+    want = std::max(want, std::min<int64_t>(kFewBlocks, (n + kBlock - 1) / kBlock));
     if (want < 1) want = 1;
     int64_t blocks = std::min<int64_t>(want, max_blocks);
     int64_t per = (n + blocks - 1) / blocks;

@@ -338,6 +338,15 @@ __device__ __forceinline__ double wave_sum_quad(const double (&v)[N])
     return s;
 }
 
+// lane `l`'s value (l the same in every lane)
+__device__ __forceinline__ double lane_value(double v, int l)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), l);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+
 // row[node] += the wave's sums of v[w], node = first_node(cell, W-1) + w: one
 // LDS add by the first lane of each row of 16 that holds a sum. Only this
 // wave adds to its row and its LDS operations run in order, so the order of

@@ -883,10 +883,13 @@ __device__ __forceinline__ int live_index(int e, int nx, unsigned mask)
 // out[i] = sum of base[b*NDEP*nx + i] over the n rows b = b0 + j * stride,
 // j in [0, n), for the live entries i of the rows in mask. Fixed order: the
 // k threads of an entry take consecutive slices of j, and their slice sums
-// are added in slice order. Called by all threads; scratch holds blockDim.x
-// doubles.
+// are added in slice order. k depends on the grid alone (the threads shared
+// by all NDEP rows, whichever of them are live), so the fused and the
+// sub-step passes' rows are summed in the same order at every row count; 1d1v
+// deposits one row and shares the threads over it (spread_rows = 1). Called
+// by all threads; scratch holds blockDim.x doubles.
 __device__ void sum_rows(const double *base, int b0, int n, int stride, int nx, unsigned mask,
-                         double *out, double *scratch)
+                         double *out, double *scratch, int spread_rows)
 {
     const int nt = blockDim.x, tid = threadIdx.x;
     const int len = NDEP * nx;
@@ -894,7 +897,7 @@ __device__ void sum_rows(const double *base, int b0, int n, int stride, int nx, 
     const size_t rs = (size_t)stride * len;
     for (int e0 = 0; e0 < E; e0 += nt) {
         const int ec = E - e0 < nt ? E - e0 : nt;
-        const int k = nt / ec;
+        const int k = spread_rows * nx < nt ? nt / (spread_rows * nx) : 1;
         const int h = tid / ec;
         const int e = e0 + (tid - h * ec);
         double s = 0.0;
@@ -904,16 +907,14 @@ __device__ void sum_rows(const double *base, int b0, int n, int stride, int nx, 
             const int r0 = (int)(((long)n * h) / k);
             const int r1 = (int)(((long)n * (h + 1)) / k);
             const double *col = base + (size_t)b0 * len + idx;
-            int b = r0;
             constexpr int B = 16;
-            for (; b + B <= r1; b += B) {
+            for (int b = r0; b < r1; b += B) {      // a short last batch adds zeros
                 double t[B];
 #pragma unroll
-                for (int u = 0; u < B; ++u) t[u] = col[(size_t)(b + u) * rs];
+                for (int u = 0; u < B; ++u) t[u] = col[(size_t)(b + u < r1 ? b + u : r1 - 1) * rs];
 #pragma unroll
-                for (int u = 0; u < B; ++u) s += t[u];
+                for (int u = 0; u < B; ++u) s += b + u < r1 ? t[u] : 0.0;
             }
-            for (; b < r1; ++b) s += col[(size_t)b * rs];
         }
         scratch[tid] = s;
         __syncthreads();
@@ -928,71 +929,83 @@ __device__ void sum_rows(const double *base, int b0, int n, int stride, int nx, 
 
 // sum_rows over the rows [b0, b1)
 __device__ __forceinline__ void sum_rows_range(const double *base, int b0, int b1, int nx,
-                                               unsigned mask, double *out, double *scratch)
+                                               unsigned mask, double *out, double *scratch,
+                                               int spread_rows = NDEP)
 {
-    sum_rows(base, b0, b1 - b0, 1, nx, mask, out, scratch);
+    sum_rows(base, b0, b1 - b0, 1, nx, mask, out, scratch, spread_rows);
 }
 
 // The first level of the field part's sum: group g of ng sums the partial
 // rows of its contiguous slice of the nblocks workgroups. (Slices of the
 // rows written on the group's own XCD, b mod ng == g, measured the same.)
 __device__ __forceinline__ void sum_group_rows(const double *part, int nblocks, int g, int ng, int nx,
-                                               unsigned mask, double *out, double *scratch)
+                                               unsigned mask, double *out, double *scratch,
+                                               int spread_rows = NDEP)
 {
     const int b0 = (int)(((long)nblocks * g) / ng), b1 = (int)(((long)nblocks * (g + 1)) / ng);
-    sum_rows_range(part, b0, b1, nx, mask, out, scratch);
+    sum_rows_range(part, b0, b1, nx, mask, out, scratch, spread_rows);
 }
 
-// (C rhs)[i] for the circulant C with first column c: sum_j c[(i - j) mod n] rhs[j],
-// in four interleaved partial sums
+// The sum of a quad's four values, (s0 + s1) + (s2 + s3), in each of its lanes
+__device__ __forceinline__ double quad_sum(double s)
+{
+    s += dpp_f64<0xB1>(s);           // quad_perm [1, 0, 3, 2]
+    return s + dpp_f64<0x4E>(s);     // quad_perm [2, 3, 0, 1]
+}
+
+// (C rhs)[i] for the circulant C with first column c, sum_j c[(i - j) mod n]
+// rhs[j], by the four lanes of a quad (all active, the same i): lane u takes
+// j = u, u + 4, ... and lane 0 what is left of n modulo 4. The products are a
+// chain of LDS reads and fused multiply-adds, so a quad is done in a quarter
+// of one lane's time, with the same four partial sums.
 __device__ __forceinline__ double circ_apply(const double *c, const double *rhs, int i, int n)
 {
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    int t = i;                                    // (i - j) mod n for j = 0
-    int j = 0;
-    for (; j + 4 <= n; j += 4) {
-        const int t1 = t == 0 ? n - 1 : t - 1;
-        const int t2 = t1 == 0 ? n - 1 : t1 - 1;
-        const int t3 = t2 == 0 ? n - 1 : t2 - 1;
-        s0 = __builtin_fma(c[t], rhs[j], s0);
-        s1 = __builtin_fma(c[t1], rhs[j + 1], s1);
-        s2 = __builtin_fma(c[t2], rhs[j + 2], s2);
-        s3 = __builtin_fma(c[t3], rhs[j + 3], s3);
-        t = t3 == 0 ? n - 1 : t3 - 1;
+    const int u = threadIdx.x & 3;
+    double s = 0.0;
+    int t = i - u, j = u;
+    if (t < 0) t += n;
+#pragma unroll 4
+    for (; j < (n & ~3); j += 4) {
+        s = __builtin_fma(c[t], rhs[j], s);
+        t -= 4;
+        if (t < 0) t += n;
     }
-    for (; j < n; ++j) {
-        s0 = __builtin_fma(c[t], rhs[j], s0);
-        t = t == 0 ? n - 1 : t - 1;
-    }
-    return (s0 + s1) + (s2 + s3);
+    if (u == 0)
+        for (; j < n; ++j) {
+            s = __builtin_fma(c[t], rhs[j], s);
+            t = t == 0 ? n - 1 : t - 1;
+        }
+    return quad_sum(s);
 }
 
-// (C^T rhs)[i] for the circulant C with first column c: sum_j c[(j - i) mod n] rhs[j]
+// (C^T rhs)[i], sum_j c[(j - i) mod n] rhs[j], in the same way
 __device__ __forceinline__ double circ_apply_t(const double *c, const double *rhs, int i, int n)
 {
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    int t = i == 0 ? 0 : n - i;                   // (j - i) mod n for j = 0
-    int j = 0;
-    for (; j + 4 <= n; j += 4) {
-        const int t1 = t + 1 == n ? 0 : t + 1;
-        const int t2 = t1 + 1 == n ? 0 : t1 + 1;
-        const int t3 = t2 + 1 == n ? 0 : t2 + 1;
-        s0 = __builtin_fma(c[t], rhs[j], s0);
-        s1 = __builtin_fma(c[t1], rhs[j + 1], s1);
-        s2 = __builtin_fma(c[t2], rhs[j + 2], s2);
-        s3 = __builtin_fma(c[t3], rhs[j + 3], s3);
-        t = t3 + 1 == n ? 0 : t3 + 1;
+    const int u = threadIdx.x & 3;
+    double s = 0.0;
+    int t = u - i, j = u;
+    if (t < 0) t += n;
+#pragma unroll 4
+    for (; j < (n & ~3); j += 4) {
+        s = __builtin_fma(c[t], rhs[j], s);
+        t += 4;
+        if (t >= n) t -= n;
     }
-    for (; j < n; ++j) {
-        s0 = __builtin_fma(c[t], rhs[j], s0);
-        t = t + 1 == n ? 0 : t + 1;
-    }
-    return (s0 + s1) + (s2 + s3);
+    if (u == 0)
+        for (; j < n; ++j) {
+            s = __builtin_fma(c[t], rhs[j], s);
+            t = t + 1 == n ? 0 : t + 1;
+        }
+    return quad_sum(s);
 }
 
-// workgroups of k_epi1d for nblocks partial rows
+// Workgroups of k_epi1d for nblocks partial rows: one while its threads hold
+// the rows in two batches of loads (no second level, fence or counter), else
+// the square root, which balances the two levels.
+constexpr int kEpiOneGroup = 64;
 int epi_groups(int nblocks)
 {
+    if (nblocks <= kEpiOneGroup) return 1;
     int g = (int)std::ceil(std::sqrt((double)nblocks));
     return g < 1 ? 1 : (g > kEpiGroupsMax ? kEpiGroupsMax : g);
 }
@@ -1019,6 +1032,7 @@ __device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g
     constexpr unsigned DEPMASK = (HP2A ? 1u << D_J2A : 0u) | (HP1 ? 1u << D_J1 : 0u) |
                                  (DEP_RHO ? 1u << D_RHO : 0u) | (HP2B ? 1u << D_J2B : 0u);
     constexpr unsigned REDMASK = DEPMASK | (WITH_J2A ? 1u << D_J2A : 0u);
+    constexpr int SPREAD = V1 ? 1 : NDEP;
     static_assert(!FAST || (HE && HP2A && HP1 && HP2B && !V1), "fused arithmetic: the fused step");
     (void)HE_PREV;
     (void)HE;
@@ -1041,37 +1055,60 @@ __device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g
     double *scratch = w3 + 6 * nx;          // [blockDim.x]
 
     if constexpr (PHASE == 1) {
-        sum_group_rows(a.part, nblocks, g, ng, nx, REDMASK, a.gpart + (size_t)g * len, scratch);
+        sum_group_rows(a.part, nblocks, g, ng, nx, REDMASK, a.gpart + (size_t)g * len, scratch, SPREAD);
         return;
     }
 
-    // every workgroup stages the fields and tables first: the one that ends up
-    // last has them in LDS without another round trip
+    // Every workgroup loads the fields and the tables it uses first (the one
+    // that ends up last then has them without another round trip), into
+    // registers, so that they arrive with the rows: nx <= kNxMax <= kBlock.
+    static_assert(kNxMax <= kBlock, "one node per thread");
+    constexpr int T0 = FAST ? T_CM0 : T_COS, TN = FAST ? 3 : 6;      // T_CM0..T_CAMP / T_COS..T_POIS
+    static_assert(T_CAMP == T_CM0 + 2 && T_POIS == T_COS + 5, "contiguous tables");
     double *G = a.grid;
-    for (int i = tid; i < nx; i += nt) {
-        sE1[i] = G[S_E1 * nx + i];
-        sE2[i] = G[S_E2 * nx + i];
-        sB[i] = G[S_B * nx + i];
+    double f_e1 = 0.0, f_e2 = 0.0, f_b = 0.0, f_t[TN];
+    if (tid < nx) {
+        f_e1 = G[S_E1 * nx + tid];
+        f_e2 = G[S_E2 * nx + tid];
+        f_b = G[S_B * nx + tid];
+#pragma unroll
+        for (int k = 0; k < TN; ++k) f_t[k] = a.tabs[(T0 + k) * nx + tid];
     }
-    for (int i = tid; i < NTAB * nx; i += nt) T[i] = a.tabs[i];
     for (int i = tid; i < len; i += nt) sRed[i] = 0.0;
+    auto stage = [&] {
+        if (tid < nx) {
+            sE1[tid] = f_e1;
+            sE2[tid] = f_e2;
+            sB[tid] = f_b;
+#pragma unroll
+            for (int k = 0; k < TN; ++k) T[(T0 + k) * nx + tid] = f_t[k];
+        }
+    };
 
-    if constexpr (PHASE == 0) {
-        // group sums of a slice of the workgroups' rows
-        sum_group_rows(a.part, nblocks, g, ng, nx, REDMASK, a.gpart + (size_t)g * len, scratch);
-        __threadfence();
+    if (PHASE == 0 && ng == 1) {
+        __syncthreads();                        // sRed is zero
+        sum_rows_range(a.part, 0, nblocks, nx, REDMASK, sRed, scratch, SPREAD);
+        stage();
         __syncthreads();
-        if (tid == 0) s_last = atomicAdd(&a.cnt[0], 1u) == (unsigned)(ng - 1);
-        __syncthreads();
-        if (!s_last) return;
-        __threadfence();
-        if (tid == 0) a.cnt[0] = 0u;            // counters are zero between launches
     } else {
-        (void)s_last;
-        __syncthreads();
+        if constexpr (PHASE == 0) {
+            // group sums of a slice of the workgroups' rows
+            sum_group_rows(a.part, nblocks, g, ng, nx, REDMASK, a.gpart + (size_t)g * len, scratch, SPREAD);
+            stage();
+            __threadfence();
+            __syncthreads();
+            if (tid == 0) s_last = atomicAdd(&a.cnt[0], 1u) == (unsigned)(ng - 1);
+            __syncthreads();
+            if (!s_last) return;
+            __threadfence();
+            if (tid == 0) a.cnt[0] = 0u;            // counters are zero between launches
+        } else {
+            (void)s_last;
+            stage();
+            __syncthreads();
+        }
+        sum_rows_range(a.gpart, 0, ng, nx, REDMASK, sRed, scratch, SPREAD);  // ends with a barrier
     }
-
-    sum_rows_range(a.gpart, 0, ng, nx, REDMASK, sRed, scratch);  // ends with a barrier
     double *r_j2a = sRed + D_J2A * nx, *r_j1 = sRed + D_J1 * nx;
     double *r_rho = sRed + D_RHO * nx, *r_j2b = sRed + D_J2B * nx;
     if constexpr (RHO_ONLY) {
@@ -1115,11 +1152,10 @@ __device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g
         for (int i = tid; i < nx; i += nt) rhs2[i] = (r_j2a[i] + r_j2b[i]) * a.dt_hp2;
         __syncthreads();
         const double rdx = 1.0 / dx;
-        for (int t = tid; t < 2 * nx; t += nt) {
-            const int g = t / nx, i = t - g * nx;
-            const double w = g == 0 ? circ_apply(T + T_CM0 * nx, rhs2, i, nx)
-                                    : circ_apply(T + T_CM1 * nx, r_j1, i, nx);
-            w3[g * nx + i] = w;
+        for (int t = tid; t < 8 * nx; t += nt) {
+            const int o = t >> 2, g = o >= nx, i = g ? o - nx : o;
+            const double w = circ_apply(T + (g ? T_CM1 : T_CM0) * nx, g ? r_j1 : rhs2, i, nx);
+            if ((t & 3) == 0) w3[o] = w;
         }
         __syncthreads();
         for (int i = tid; i < nx; i += nt) {
@@ -1143,7 +1179,10 @@ __device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g
         __syncthreads();
         // HB of this step and (a.more) of the next one: the weak curl of B once
         const double times = a.more ? 2.0 * coef : coef;
-        for (int i = tid; i < nx; i += nt) hc[i] = circ_apply(T + T_CAMP * nx, sB, i, nx);
+        for (int t = tid; t < 4 * nx; t += nt) {
+            const double w = circ_apply(T + T_CAMP * nx, sB, t >> 2, nx);
+            if ((t & 3) == 0) hc[t >> 2] = w;
+        }
         __syncthreads();
         for (int i = tid; i < nx; i += nt) sE2[i] = __builtin_fma(times, hc[i], sE2[i]);
         __syncthreads();
@@ -1762,25 +1801,46 @@ __global__ void __launch_bounds__(kBlock) k_boris_epi(PassArgs a, int nblocks)
     double *scratch = w3 + 6 * nx;          // [blockDim.x]
     double *G = a.grid;
     const int se1 = KIND == BE_STAGGER ? S_E1 : S_E1M, se2 = KIND == BE_STAGGER ? S_E2 : S_E2M;
-    for (int i = tid; i < nx; i += nt) {
-        sE1[i] = G[se1 * nx + i];
-        sE2[i] = G[se2 * nx + i];
-        sB[i] = G[S_B * nx + i];
+    // loaded into registers first, so that they arrive with the rows (as k_epi1d)
+    constexpr int TN = 5;                   // T_COS .. T_AMP
+    static_assert(T_AMP == T_COS + TN - 1, "contiguous tables");
+    double f_e1 = 0.0, f_e2 = 0.0, f_b = 0.0, f_t[TN];
+    if (tid < nx) {
+        f_e1 = G[se1 * nx + tid];
+        f_e2 = G[se2 * nx + tid];
+        f_b = G[S_B * nx + tid];
+#pragma unroll
+        for (int k = 0; k < TN; ++k) f_t[k] = a.tabs[(T_COS + k) * nx + tid];
     }
-    for (int i = tid; i < NTAB * nx; i += nt) T[i] = a.tabs[i];
     for (int i = tid; i < len; i += nt) sRed[i] = 0.0;
+    auto stage = [&] {
+        if (tid < nx) {
+            sE1[tid] = f_e1;
+            sE2[tid] = f_e2;
+            sB[tid] = f_b;
+#pragma unroll
+            for (int k = 0; k < TN; ++k) T[(T_COS + k) * nx + tid] = f_t[k];
+        }
+    };
 
     const int ng = gridDim.x, g = blockIdx.x;
-    const int b0 = (int)(((long)nblocks * g) / ng), b1 = (int)(((long)nblocks * (g + 1)) / ng);
-    sum_rows_range(a.part, b0, b1, nx, REDMASK, a.gpart + (size_t)g * len, scratch);
-    __threadfence();
-    __syncthreads();
-    if (tid == 0) s_last = atomicAdd(&a.cnt[0], 1u) == (unsigned)(ng - 1);
-    __syncthreads();
-    if (!s_last) return;
-    __threadfence();
-    if (tid == 0) a.cnt[0] = 0u;
-    sum_rows_range(a.gpart, 0, ng, nx, REDMASK, sRed, scratch);
+    if (ng == 1) {
+        __syncthreads();                    // sRed is zero
+        sum_rows_range(a.part, 0, nblocks, nx, REDMASK, sRed, scratch);
+        stage();
+        __syncthreads();
+    } else {
+        sum_group_rows(a.part, nblocks, g, ng, nx, REDMASK, a.gpart + (size_t)g * len, scratch);
+        stage();
+        __threadfence();
+        __syncthreads();
+        if (tid == 0) s_last = atomicAdd(&a.cnt[0], 1u) == (unsigned)(ng - 1);
+        __syncthreads();
+        if (!s_last) return;
+        __threadfence();
+        if (tid == 0) a.cnt[0] = 0u;
+        sum_rows_range(a.gpart, 0, ng, nx, REDMASK, sRed, scratch);
+    }
     double *r_j1 = sRed + D_J1 * nx, *r_j2 = sRed + D_J2A * nx;
     if constexpr (KIND == BE_J) {
         for (int i = tid; i < nx; i += nt) {
@@ -3108,27 +3168,58 @@ __device__ __forceinline__ void adj_epi_body(const AdjArgs &A, int nblocks, int 
     double *scratch = bend + nx;            // [blockDim.x]
     double *G = A.agrid;
 
-    for (int i = tid; i < nx; i += nt) {
-        lE1[i] = G[A_E1 * nx + i];
-        lE2[i] = G[A_E2 * nx + i];
-        lB[i] = G[A_B * nx + i];
-        bend[i] = A.bend ? A.bend[i] : 0.0;
+    // loaded into registers first, so that they arrive with the rows (as
+    // k_epi1d): the cotangents, B at the step's end, E2 of the step's HE pair
+    // (into the slots of tables not used here) and the circulant columns
+    static_assert(T_CPOIS == T_CM0 + 4, "contiguous tables");
+    constexpr int TN = KIND == AE_POIS ? 0 : 4;
+    double *sE2f = T + T_COS * nx, *sE2c = T + T_SIN * nx;
+    double f_l[3] = {0.0, 0.0, 0.0}, f_bend = 0.0, f_e2f = 0.0, f_e2c = 0.0, f_t[5];
+    if (tid < nx) {
+        f_l[0] = G[A_E1 * nx + tid];
+        f_l[1] = G[A_E2 * nx + tid];
+        f_l[2] = G[A_B * nx + tid];
+        if (A.bend) f_bend = A.bend[tid];
+        if (KIND != AE_POIS && A.fields) {
+            f_e2f = A.fields[H_E2 * nx + tid];
+            f_e2c = A.fields[H_E2P * nx + tid];
+        }
+#pragma unroll
+        for (int k = 0; k < 5; ++k)
+            if (k < TN || KIND == AE_POIS) f_t[k] = a.tabs[(T_CM0 + k) * nx + tid];
     }
-    for (int i = tid; i < NTAB * nx; i += nt) T[i] = a.tabs[i];
     for (int i = tid; i < len; i += nt) red[i] = 0.0;
-    __syncthreads();
+    auto stage = [&] {
+        if (tid < nx) {
+            lE1[tid] = f_l[0];
+            lE2[tid] = f_l[1];
+            lB[tid] = f_l[2];
+            bend[tid] = f_bend;
+            sE2f[tid] = f_e2f;
+            sE2c[tid] = f_e2c;
+#pragma unroll
+            for (int k = 0; k < 5; ++k)
+                if (k < TN || KIND == AE_POIS) T[(T_CM0 + k) * nx + tid] = f_t[k];
+        }
+    };
 
     constexpr unsigned MASK = KIND == AE_TAIL ? (1u << AR_E1) | (1u << AR_E2) | (1u << AR_SCAL)
                               : KIND == AE_POIS ? 0u
                                                 : (1u << AR_E1) | (1u << AR_E2) | (1u << AR_B) |
                                                       (1u << AR_SCAL);
-    if constexpr (MASK != 0u) {
+    if (MASK == 0u || (PHASE == 0 && ng == 1)) {
+        __syncthreads();                        // red is zero
+        if constexpr (MASK != 0u) sum_rows_range(a.part, 0, nblocks, nx, MASK, red, scratch);
+        stage();
+        __syncthreads();
+    } else {
         // PHASE 1: only this workgroup's slice sum; PHASE 2: only the rest (a
         // later launch, no fences or counters); PHASE 0: both, as one launch
         if constexpr (PHASE != 2) {
             const int b0 = (int)(((long)nblocks * gb) / ng), b1 = (int)(((long)nblocks * (gb + 1)) / ng);
             sum_rows_range(a.part, b0, b1, nx, MASK, a.gpart + (size_t)gb * len, scratch);
             if constexpr (PHASE == 1) return;
+            stage();
             __threadfence();
             __syncthreads();
             if (tid == 0) s_last = atomicAdd(&a.cnt[0], 1u) == (unsigned)(ng - 1);
@@ -3138,10 +3229,11 @@ __device__ __forceinline__ void adj_epi_body(const AdjArgs &A, int nblocks, int 
             if (tid == 0) a.cnt[0] = 0u;
         } else {
             (void)s_last;
+            stage();
+            __syncthreads();
         }
         sum_rows_range(a.gpart, 0, ng, nx, MASK, red, scratch);
     }
-    __syncthreads();
     const double *dE1 = red + AR_E1 * nx, *dE2 = red + AR_E2 * nx, *dB = red + AR_B * nx;
     const double c = a.dt_he;
     const double coef = c / dx;
@@ -3151,21 +3243,27 @@ __device__ __forceinline__ void adj_epi_body(const AdjArgs &A, int nblocks, int 
     //   H = compute_e_from_b!:  -(1/dx) lambda_E2 . (c/dx) W B = -(1/dx) (c/dx) (W^T lambda_E2) . B
     //   L = w/2 dx B.M1 B:      w/2 B.M1 B
     double gdx = 0.0;
-    const double *E2f = A.fields ? A.fields + H_E2 * nx : nullptr;
-    const double *E2c = A.fields ? A.fields + H_E2P * nx : nullptr;
-    // grid dot products: wave 0's lanes take nodes j = lane, lane + 64, ...,
-    // and a butterfly adds the lanes in a fixed order (the sum is the same in
-    // every lane of wave 0; call from all of wave 0 only)
+    const double *E2f = sE2f, *E2c = sE2c;
+    // grid dot products: wave 0's lanes take nodes j = lane, lane + 64, ...
+    // (call from all of wave 0 only); sum_lanes adds the lanes of up to three
+    // of them in a fixed order, the k-th sum to out[k] in every lane
     auto dot_d = [&](const double *lb, const double *e) {      // lb . D e, D e[j] = e[j-1] - e[j]
         double r = 0.0;
         for (int j = tid; j < nx; j += kWave) r += lb[j] * (e[j == 0 ? nx - 1 : j - 1] - e[j]);
-        return wave_sum(r);
+        return r;
     };
     auto dot = [&](const double *u, const double *v) {
         double r = 0.0;
         for (int j = tid; j < nx; j += kWave) r += u[j] * v[j];
-        return wave_sum(r);
+        return r;
     };
+    auto sum_lanes = [&](double (&r)[3]) {
+        const double s = wave_sum_quad<3>(r);
+        r[0] = lane_value(s, 0);
+        r[1] = lane_value(s, 32);                  // rows 0, 2 and 1 hold the sums 0, 1 and 2
+        r[2] = lane_value(s, 16);
+    };
+    static_assert(quad_value(0) == 0 && quad_value(2) == 1 && quad_value(1) == 2, "rows of the sums");
     if (KIND != AE_POIS && tid == 0) {
         G[A_LOSS * nx + AS_DX] = G[A_LOSS * nx + AS_DX] + red[AR_SCAL * nx + 0];
         G[A_LOSS * nx + AS_MOD] = G[A_LOSS * nx + AS_MOD] + red[AR_SCAL * nx + 1];
@@ -3185,7 +3283,10 @@ __device__ __forceinline__ void adj_epi_body(const AdjArgs &A, int nblocks, int 
         }
         __syncthreads();
         adj_b_from_e(tmp, 1.0, bend, nx);
-        for (int i = tid; i < nx; i += nt) G[A_NU * nx + i] = circ_apply(T + T_CPOIS * nx, tmp, i, nx);
+        for (int t = tid; t < 4 * nx; t += nt) {
+            const double w = circ_apply(T + T_CPOIS * nx, tmp, t >> 2, nx);
+            if ((t & 3) == 0) G[A_NU * nx + (t >> 2)] = w;
+        }
         return;
     }
     if constexpr (KIND == AE_STEP || KIND == AE_HEAD) {
@@ -3197,13 +3298,17 @@ __device__ __forceinline__ void adj_epi_body(const AdjArgs &A, int nblocks, int 
         }
         __syncthreads();
         if (tid < kWave) {
-            const double r = dot_d(lB, E2f);
-            if (tid == 0) gdx = gdx - (coef / dx) * r;
+            double r[3] = {dot_d(lB, E2f), 0.0, 0.0};
+            sum_lanes(r);
+            if (tid == 0) gdx = gdx - (coef / dx) * r[0];
         }
         adj_b_from_e(lE2, coef, lB, nx);                       // U of the next step's HE
     }
     if constexpr (KIND == AE_HEAD) {
-        for (int i = tid; i < nx; i += nt) wA[i] = circ_apply_t(T + T_CAMP * nx, lE2, i, nx);
+        for (int t = tid; t < 4 * nx; t += nt) {
+            const double w = circ_apply_t(T + T_CAMP * nx, lE2, t >> 2, nx);
+            if ((t & 3) == 0) wA[t >> 2] = w;
+        }
         __syncthreads();                                        // H of the first step
         for (int i = tid; i < nx; i += nt) {
             lB[i] = lB[i] + coef * wA[i];
@@ -3213,9 +3318,10 @@ __device__ __forceinline__ void adj_epi_body(const AdjArgs &A, int nblocks, int 
         }
         __syncthreads();
         if (tid < kWave) {
-            const double r = dot(wA, bend);                    // (W^T lambda_E2) . B_0
+            double r[3] = {dot(wA, bend), 0.0, 0.0};           // (W^T lambda_E2) . B_0
+            sum_lanes(r);
             if (tid == 0) {
-                gdx = gdx - (coef / dx) * r;
+                gdx = gdx - (coef / dx) * r[0];
                 G[A_LOSS * nx + AS_DX] = G[A_LOSS * nx + AS_DX] + gdx;
             }
         }
@@ -3227,11 +3333,11 @@ __device__ __forceinline__ void adj_epi_body(const AdjArgs &A, int nblocks, int 
         __syncthreads();
         // W^T lambda_E2, M1 B_end and M1^-1 lambda_E1, each a matrix-vector
         // product with the circulant's first column
-        for (int t = tid; t < 3 * nx; t += nt) {
-            const int k = t / nx, i = t - k * nx;
-            if (k == 0) wA[i] = circ_apply_t(T + T_CAMP * nx, lE2, i, nx);
-            else if (k == 1) wM[i] = circ_apply(T + T_CMASS1 * nx, bend, i, nx);
-            else w1[i] = circ_apply(T + T_CM1 * nx, lE1, i, nx);
+        for (int t = tid; t < 12 * nx; t += nt) {
+            const int o = t >> 2, k = (o >= nx) + (o >= 2 * nx), i = o - k * nx;
+            const double w = k == 0 ? circ_apply_t(T + T_CAMP * nx, lE2, i, nx)
+                                    : circ_apply(T + (k == 1 ? T_CMASS1 : T_CM1) * nx, k == 1 ? bend : lE1, i, nx);
+            if ((t & 3) == 0) wA[o] = w;              // wA, wM and w1 one behind the other
         }
         __syncthreads();
         const double wl = A.wloss;
@@ -3245,20 +3351,23 @@ __device__ __forceinline__ void adj_epi_body(const AdjArgs &A, int nblocks, int 
         }
         __syncthreads();
         if (tid < kWave) {
-            const double r = dot(bend, wM), rh = dot(wA, bend);
-            const double rd = dot_d(lB, E2c);
+            double r[3] = {dot(bend, wM), dot(wA, bend), dot_d(lB, E2c)};
+            sum_lanes(r);
             if (tid == 0) {
-                G[A_LOSS * nx] = G[A_LOSS * nx] + wl * 0.5 * (r * dx);
-                gdx = gdx + wl * 0.5 * r - (KIND == AE_STEP ? 2.0 : 1.0) * (coef / dx) * rh;
-                gdx = gdx - (coef / dx) * rd;
+                G[A_LOSS * nx] = G[A_LOSS * nx] + wl * 0.5 * (r[0] * dx);
+                gdx = gdx + wl * 0.5 * r[0] - (KIND == AE_STEP ? 2.0 : 1.0) * (coef / dx) * r[1];
+                gdx = gdx - (coef / dx) * r[2];
                 G[A_LOSS * nx + AS_DX] = G[A_LOSS * nx + AS_DX] + gdx;
             }
         }
         adj_b_from_e(lE2, coef, lB, nx);                       // U of this step's HE
         for (int i = tid; i < nx; i += nt) lE2[i] = lE2[i] + dE2[i];
         __syncthreads();
+        for (int t = tid; t < 4 * nx; t += nt) {
+            const double w = circ_apply(T + T_CM0 * nx, lE2, t >> 2, nx);
+            if ((t & 3) == 0) G[A_MU2 * nx + (t >> 2)] = -(c / dx) * w;
+        }
         for (int i = tid; i < nx; i += nt) {
-            G[A_MU2 * nx + i] = -(c / dx) * circ_apply(T + T_CM0 * nx, lE2, i, nx);
             G[A_E1 * nx + i] = lE1[i];
             G[A_E2 * nx + i] = lE2[i];
             G[A_B * nx + i] = lB[i];
