@@ -302,7 +302,9 @@ namespace gl {
 // solver's own stream: compute_e_from_b!, compute_b_from_e!, E -= M1^{-1} j
 // (compute_e_from_j!) and compute_rho_from_e! (maxwell_2d_fem.jl:370-499)
 hipStream_t m2d_stream(gempic_maxwell2d *m);
-void m2d_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *const *e);
+// (with es, where m2d_fused: also es = E before + E after)
+void m2d_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *const *e,
+                  double *const *es = nullptr);
 void m2d_b_from_e(gempic_maxwell2d *m, double dt, double *const *e, double *const *b);
 void m2d_e_from_j(gempic_maxwell2d *m, const double *j, int component, double *e);
 // j = (sum of the partial grids part2[0 .. splits - 1], in order) * scale,
@@ -310,5 +312,11 @@ void m2d_e_from_j(gempic_maxwell2d *m, const double *j, int component, double *e
 // queued) where the grid takes the general path (m2d_e_from_j)
 bool m2d_e_from_parts(gempic_maxwell2d *m, const double *part2, int splits, double scale, double *j,
                       int component, double *e);
+// whether the grid takes the row and column field kernels
+bool m2d_fused(const gempic_maxwell2d *m);
+// the same for all three components (m2d_fused grids): their split sums at
+// part2[split][component][node], scale[c] each
+void m2d_e_from_parts3(gempic_maxwell2d *m, const double *part2, int splits, const double *scale,
+                       double *const *j, double *const *e);
 void m2d_rho_from_e(gempic_maxwell2d *m, double *const *e, double *rho);
 }  // namespace gl

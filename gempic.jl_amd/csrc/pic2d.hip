@@ -665,13 +665,45 @@ __global__ void __launch_bounds__(kFieldThreads) k_fj_rows(Field2 f, const doubl
     conv_rows(jr, kk, rows, nx, tmp + (size_t)r0 * nx, nx);
 }
 
+// k_fj_rows for the components of the fused 2D3V step, blockIdx.y each: the
+// currents' split sums lie at part2[split][component][node]
+struct FieldJ3 {
+    double scale[3];
+    const double *kx[3];
+    double *jout[3];
+    double *tmp[3];
+};
+
+__global__ void __launch_bounds__(kFieldThreads) k_fj_rows3(Field2 f, const double *part2, int splits, FieldJ3 a)
+{
+    extern __shared__ __align__(16) double lds[];
+    const int nx = f.nx, nn = nx * f.ny, c = blockIdx.y;
+    const int r0 = blockIdx.x * kFieldRows, rows = min(kFieldRows, f.ny - r0);
+    double *jr = lds, *kk = lds + kFieldRows * nx;
+    const double *kx = a.kx[c];
+    for (int m = threadIdx.x; m < nx; m += blockDim.x) kk[m] = kx[m];
+    for (int t = threadIdx.x; t < rows * nx; t += blockDim.x) {
+        const int k = r0 * nx + t;
+        double v = 0.0;
+#pragma unroll 16
+        for (int sp = 0; sp < splits; ++sp) v += part2[((size_t)sp * 3 + c) * nn + k];
+        v = v * a.scale[c];
+        a.jout[c][k] = v;
+        jr[t] = v;
+    }
+    __syncthreads();
+    conv_rows(jr, kk, rows, nx, a.tmp[c] + (size_t)r0 * nx, nx);
+}
+
 // second kernel of both updates: the columns c0 .. c0 + cols - 1 of tmp
 // (component blockIdx.y), their inverse mass along y, e = e + coef w
-// (coef = dt: k_axpy; coef = -1: k_sub, bitwise e - w)
+// (coef = dt: k_axpy; coef = -1: k_sub, bitwise e - w); with es, also
+// es = e before + e after
 struct FieldCols {
     const double *tmp[3];
     const double *ky[3];
     double *e[3];
+    double *es[3];
 };
 
 __global__ void __launch_bounds__(kFieldThreads) k_f_cols(Field2 f, FieldCols a, double coef)
@@ -698,7 +730,9 @@ __global__ void __launch_bounds__(kFieldThreads) k_f_cols(Field2 f, FieldCols a,
             u = u == 0 ? ny - 1 : u - 1;
         }
         const size_t k = (size_t)j * nx + c0 + cc;
-        e[k] = e[k] + coef * acc;
+        const double e0 = e[k], e1 = e0 + coef * acc;
+        e[k] = e1;
+        if (a.es[c]) a.es[c][k] = e0 + e1;
     }
 }
 
@@ -1044,7 +1078,9 @@ size_t nn2(const gempic_maxwell2d *m) { return (size_t)m->nx * m->ny; }
 // (used by the 2D3V splitting, split2d.hip)
 hipStream_t gl::m2d_stream(gempic_maxwell2d *m) { return m->stream; }
 
-void gl::m2d_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *const *e)
+bool gl::m2d_fused(const gempic_maxwell2d *m) { return m->fused; }
+
+void gl::m2d_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *const *e, double *const *es)
 {
     const Field2 f = m->f();
     if (m->fused) {
@@ -1052,7 +1088,8 @@ void gl::m2d_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *
         FieldRowsB ra{{b[0], b[1], b[2]}, {m->buf(9), m->buf(10), m->buf(11)}};
         hipLaunchKernelGGL(k_fb_rows, dim3((m->ny + kFieldRows - 1) / kFieldRows, 3), dim3(kFieldThreads),
                            fb_rows_lds(m), m->stream, f, t, ra);
-        FieldCols ca{{m->buf(9), m->buf(10), m->buf(11)}, {t.k0y, t.k1y, t.k0y}, {e[0], e[1], e[2]}};
+        FieldCols ca{{m->buf(9), m->buf(10), m->buf(11)}, {t.k0y, t.k1y, t.k0y}, {e[0], e[1], e[2]},
+                     {es ? es[0] : nullptr, es ? es[1] : nullptr, es ? es[2] : nullptr}};
         hipLaunchKernelGGL(k_f_cols, dim3((m->nx + kFieldCols - 1) / kFieldCols, 3), dim3(kFieldThreads),
                            f_cols_lds(m), m->stream, f, ca, dt);
         return;
@@ -1093,10 +1130,25 @@ bool gl::m2d_e_from_parts(gempic_maxwell2d *m, const double *part2, int splits, 
                        sizeof(double) * (size_t)(kFieldRows + 1) * m->nx, m->stream, f, part2, splits, scale,
                        component == 1 ? t.k1x : t.k0x, j, m->buf(12));
     FieldCols ca{{m->buf(12), nullptr, nullptr}, {component == 2 ? t.k1y : t.k0y, nullptr, nullptr},
-                 {e, nullptr, nullptr}};
+                 {e, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
     hipLaunchKernelGGL(k_f_cols, dim3((m->nx + kFieldCols - 1) / kFieldCols, 1), dim3(kFieldThreads),
                        f_cols_lds(m), m->stream, f, ca, -1.0);
     return true;
+}
+
+void gl::m2d_e_from_parts3(gempic_maxwell2d *m, const double *part2, int splits, const double *scale,
+                           double *const *j, double *const *e)
+{
+    const Field2 f = m->f();
+    const FieldTabs t = field_tabs(m);
+    FieldJ3 a{{scale[0], scale[1], scale[2]}, {t.k1x, t.k0x, t.k0x}, {j[0], j[1], j[2]},
+              {m->buf(9), m->buf(10), m->buf(11)}};
+    hipLaunchKernelGGL(k_fj_rows3, dim3((m->ny + kFieldRows - 1) / kFieldRows, 3), dim3(kFieldThreads),
+                       sizeof(double) * (size_t)(kFieldRows + 1) * m->nx, m->stream, f, part2, splits, a);
+    FieldCols ca{{m->buf(9), m->buf(10), m->buf(11)}, {t.k0y, t.k1y, t.k0y}, {e[0], e[1], e[2]},
+                 {nullptr, nullptr, nullptr}};
+    hipLaunchKernelGGL(k_f_cols, dim3((m->nx + kFieldCols - 1) / kFieldCols, 3), dim3(kFieldThreads),
+                       f_cols_lds(m), m->stream, f, ca, -1.0);
 }
 
 void gl::m2d_rho_from_e(gempic_maxwell2d *m, double *const *e, double *rho)

@@ -669,6 +669,8 @@ __global__ void k_s2_out(double *aos, int64_t ld, int64_t n, S2Perm pm)
     }
 }
 
+#include "step2d.hpp"
+
 }  // namespace
 
 struct gempic_splitting2d {
@@ -693,6 +695,15 @@ struct gempic_splitting2d {
     // 360 us once the order is gone. Over 200 steps: 2.33 ms per step
     // unsorted, 2.96 ms sorting every 20 steps, 2.54 every 50.
     int64_t sort_interval = 0, steps_since_sort = 0;
+    // the fused step (step2d.hpp): its LDS layout, work arrays and the state
+    // of the binning by strip
+    bool f2 = false;                        // the grid takes it
+    bool f2_slow = false;                   // too many listed particles: the operators' passes instead
+    int f2_s = 0, f2_hr = 0, f2_strips = 1, f2_h = 0, f2_m = 0, f2_ntiles = 0;
+    bool binned = false;
+    int64_t steps_since_bin = 0, f2_steps = 0;
+    double *d_fpart = nullptr, *d_es[3] = {}, *d_stray = nullptr;
+    int *d_bin = nullptr, *d_wg = nullptr, *d_list = nullptr;
 };
 
 namespace {
@@ -850,17 +861,171 @@ int s2_sort(gempic_splitting2d *h)
     return GEMPIC_OK;
 }
 
+// Steps between binnings by strip. Particles of the Landau configuration
+// drift 0.25 cells (rms) a step, 2.5 in ten, within the 5 rows to spare.
+constexpr int kBinEvery = 10;
+// The fused step's listed particles, of all in a step, from which the
+// operators' passes are the faster way: FIXME
+constexpr int kF2ListedMost = 32;
+
 int s2_finish(gempic_splitting2d *h)
 {
     S2_TRY("2D3V splitting", hipStreamSynchronize(h->stream));
-    int err = 0;
-    S2_TRY("2D3V splitting", hipMemcpy(&err, h->d_err, sizeof(int), hipMemcpyDeviceToHost));
+    int flags[2] = {0, 0};                  // the error bits, the fused steps' listed particles
+    S2_TRY("2D3V splitting", hipMemcpy(flags, h->d_err, sizeof(flags), hipMemcpyDeviceToHost));
+    const int err = flags[0];
+    if (h->f2_steps > 0) {
+        if ((double)flags[1] * kF2ListedMost > (double)h->n * (double)h->f2_steps) h->f2_slow = true;
+        h->f2_steps = 0;
+    }
+    if (flags[0] || flags[1]) S2_TRY("2D3V splitting", hipMemset(h->d_err, 0, sizeof(flags)));
     if (err) {
-        S2_TRY("2D3V splitting", hipMemset(h->d_err, 0, sizeof(int)));
         if (err & E_INEXACT)
             return abi_fail(GEMPIC_ERR_INEXACT, "InexactError: ceil(Int, x) of a non-finite or out-of-range position");
         return abi_fail(GEMPIC_ERR_INEXACT, "a particle crossed more than 65536 cells in one push");
     }
+    return GEMPIC_OK;
+}
+
+// The fused step's LDS layout (step2d.hpp) for a grid: the whole grid where
+// nine fit, else strips with a fifth of the rows to spare on each side; false
+// where a strip would be narrower than the rows to spare.
+bool f2_layout(gempic_splitting2d *h)
+{
+    const int P = h->p;
+    if (!m2d_fused(h->m) || h->n >= (int64_t)1 << 29) return false;
+    h->f2_s = h->nx + P + 1 + ((20 - (h->nx + P + 1) % 16) % 16);   // = 4 (mod 16): see grid_stride
+    const int most = (int)(kF2Lds / (sizeof(double) * 9 * (size_t)h->f2_s));
+    if (h->ny + P + 1 <= most) {
+        h->f2_strips = 1;
+        h->f2_h = h->ny;
+        h->f2_m = 0;
+        h->f2_hr = h->ny + P + 1;
+        return true;
+    }
+    const int rows = most - P - 1;
+    int m = rows / 5;
+    if (m < 2) return false;
+    const int strips = (h->ny + rows - 2 * m - 1) / (rows - 2 * m);
+    const int hh = (h->ny + strips - 1) / strips;
+    m = (rows - hh) / 2;
+    if (strips > kF2StripsMax || hh < m || hh + 2 * m > h->ny) return false;
+    h->f2_strips = strips;
+    h->f2_h = hh;
+    h->f2_m = m;
+    h->f2_hr = hh + 2 * m + P + 1;
+    return true;
+}
+
+size_t f2_shmem(const gempic_splitting2d *h, int mode)
+{
+    return sizeof(double) * (size_t)((mode & F2_HE ? 9 : 6) * h->f2_s * h->f2_hr);
+}
+
+const void *f2_kernel(int p, int mode, bool listed = false)
+{
+#define F2K(P)                                                                                    \
+    if (listed)                                                                                   \
+        return mode == F2_ALL ? (const void *)k_f2_listed<P, F2_ALL>                              \
+               : mode == F2_FIRST ? (const void *)k_f2_listed<P, F2_FIRST>                        \
+                                  : (const void *)k_f2_listed<P, F2_SECOND>;                      \
+    return mode == F2_ALL ? (const void *)k_step2d<P, F2_ALL>                                     \
+           : mode == F2_FIRST ? (const void *)k_step2d<P, F2_FIRST>                               \
+                              : (const void *)k_step2d<P, F2_SECOND>;
+    if (p == 1) { F2K(1) }
+    if (p == 2) { F2K(2) }
+    F2K(3)
+#undef F2K
+}
+
+F2Args f2_args(gempic_splitting2d *h, double dt)
+{
+    F2Args a{};
+    a.n = h->n;
+    a.nx = h->nx;
+    a.ny = h->ny;
+    a.s = h->f2_s;
+    a.hr = h->f2_hr;
+    a.strips = h->f2_strips;
+    a.h = h->f2_h;
+    a.m = h->f2_m;
+    a.wg = h->d_wg;
+    a.xmin = h->xmin;
+    a.ymin = h->ymin;
+    a.dx = h->dx;
+    a.dy = h->dy;
+    a.rdx = 1.0 / h->dx;
+    a.rdy = 1.0 / h->dy;
+    a.Lx = h->Lx;
+    a.Ly = h->Ly;
+    a.charge = h->charge;
+    a.cw = h->cw;
+    a.qm = h->qm;
+    a.dt = dt;
+    a.dt_half = 0.5 * dt;
+    a.x1 = h->d_p[0];
+    a.x2 = h->d_p[1];
+    a.v1 = h->d_p[2];
+    a.v2 = h->d_p[3];
+    a.v3 = h->d_p[4];
+    a.w = h->d_p[5];
+    for (int c = 0; c < 3; ++c) a.b[c] = h->d_b[c];
+    a.part = h->d_fpart;
+    a.stray = h->d_stray;
+    a.list = h->d_list;
+    a.flags = h->d_err;
+    return a;
+}
+
+// particles by strip, and the ranges of the particle workgroups
+int f2_bin(gempic_splitting2d *h)
+{
+    F2Args a = f2_args(h, 0.0);
+    const int64_t chunk = ((h->n + h->blocks - h->f2_strips - 1) / (h->blocks - h->f2_strips) + kWave - 1) / kWave * kWave;
+    hipLaunchKernelGGL(k_bin_count, dim3(h->f2_ntiles), dim3(1024), 0, h->stream, a, h->f2_ntiles, h->d_bin);
+    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, h->stream, a, h->f2_ntiles, h->d_bin, h->blocks, chunk,
+                       h->d_wg);
+    S2Perm pm{};
+    for (int r = 0; r < 6; ++r) {
+        pm.src[r] = h->d_p[r];
+        pm.dst[r] = h->d_p2[r];
+    }
+    pm.id = h->d_id;
+    pm.id_dst = h->d_id2;
+    hipLaunchKernelGGL(k_bin_scatter, dim3(h->f2_ntiles), dim3(1024), 0, h->stream, a, h->f2_ntiles,
+                       (const int *)h->d_bin, pm);
+    S2_TRY("2D3V binning", hipGetLastError());
+    for (int r = 0; r < 6; ++r) std::swap(h->d_p[r], h->d_p2[r]);
+    std::swap(h->d_id, h->d_id2);
+    h->binned = true;
+    h->steps_since_bin = 0;
+    return GEMPIC_OK;
+}
+
+// a particle pass of the fused step with the E fields `e`, its current sums
+// into j_dofs, E -= their inverse mass
+int f2_pass(gempic_splitting2d *h, int mode, double dt, double *const *e)
+{
+    F2Args a = f2_args(h, dt);
+    for (int c = 0; c < 3; ++c) a.e[c] = e[c];
+    int nblk = h->blocks;
+    const int nt = f2_threads(h->p);
+    if (a.strips == 1) {
+        nblk = (int)std::max<int64_t>(1, std::min<int64_t>(nblk, (h->n + nt - 1) / nt));
+        a.chunk = ((h->n + nblk - 1) / nblk + kWave - 1) / kWave * kWave;
+    }
+    void *args[] = {&a};
+    S2_TRY("2D3V fused pass", hipLaunchKernel(f2_kernel(h->p, mode), dim3(nblk), dim3(nt), args,
+                                              f2_shmem(h, mode), h->stream));
+    S2_TRY("2D3V listed particles", hipLaunchKernel(f2_kernel(h->p, mode, true), dim3(64), dim3(256), args, 0,
+                                                    h->stream));
+    const int nn = h->nx * h->ny, splits = std::min(nblk, kSplits2);
+    double *part2 = h->d_fpart + (size_t)h->blocks * 3 * h->f2_hr * h->nx;
+    hipLaunchKernelGGL(k_f2_reduce, dim3((unsigned)((nn + 255) / 256), (unsigned)splits, 3), dim3(256), 0, h->stream,
+                       a, h->p, nblk, part2);
+    S2_TRY("2D3V current sum", hipGetLastError());
+    const double scale[3] = {1.0, 1.0, a.dt_half};
+    m2d_e_from_parts3(h->m, part2, splits, scale, h->d_j, h->d_e);
     return GEMPIC_OK;
 }
 
@@ -955,10 +1120,24 @@ int gempic_splitting2d_create(int64_t nx, int64_t ny, double xmin, double xmax, 
     }
     al((void **)&h->d_rho, sizeof(double) * nn);
     al((void **)&h->d_part, sizeof(double) * nn * (size_t)(h->blocks + kSplits2));
-    al((void **)&h->d_err, sizeof(int));
+    al((void **)&h->d_err, 3 * sizeof(int));
+    h->f2 = f2_layout(h) && h->blocks > 2 * h->f2_strips;
+    if (h->f2) {
+        h->f2_ntiles = (int)((np + kBinTile - 1) / kBinTile);
+        for (int c = 0; c < 3; ++c) al((void **)&h->d_es[c], sizeof(double) * nn);
+        al((void **)&h->d_stray, sizeof(double) * 3 * nn);
+        al((void **)&h->d_fpart, sizeof(double) * 3 * ((size_t)h->blocks * h->f2_hr * nx + (size_t)kSplits2 * nn));
+        al((void **)&h->d_bin, sizeof(int) * (size_t)h->f2_strips * h->f2_ntiles);
+        al((void **)&h->d_wg, sizeof(int) * 3 * (size_t)h->blocks);
+        al((void **)&h->d_list, sizeof(int) * np);
+        if (e == hipSuccess) e = hipMemset(h->d_stray, 0, sizeof(double) * 3 * nn);
+        for (int mode : {F2_ALL, F2_FIRST, F2_SECOND})
+            if (e == hipSuccess && f2_shmem(h, mode) > 65536)
+                e = hipFuncSetAttribute(f2_kernel(degree, mode), hipFuncAttributeMaxDynamicSharedMemorySize, kF2Lds);
+    }
     al((void **)&h->d_count, sizeof(int) * nn);
     al((void **)&h->d_cursor, sizeof(int) * nn);
-    if (e == hipSuccess) e = hipMemset(h->d_err, 0, sizeof(int));
+    if (e == hipSuccess) e = hipMemset(h->d_err, 0, 3 * sizeof(int));
     for (int c = 0; c < 3 && e == hipSuccess; ++c) {
         e = hipMemset(h->d_e[c], 0, sizeof(double) * nn);
         if (e == hipSuccess) e = hipMemset(h->d_b[c], 0, sizeof(double) * nn);
@@ -994,7 +1173,8 @@ int gempic_splitting2d_destroy(gempic_splitting2d *h)
     }
     void *bufs[] = {h->d_id, h->d_id2, h->d_e[0], h->d_e[1], h->d_e[2], h->d_b[0], h->d_b[1], h->d_b[2],
                     h->d_j[0], h->d_j[1], h->d_j[2], h->d_rho, h->d_part, h->d_stage, h->d_err,
-                    h->d_count, h->d_cursor};
+                    h->d_count, h->d_cursor, h->d_es[0], h->d_es[1], h->d_es[2], h->d_stray, h->d_fpart,
+                    h->d_bin, h->d_wg, h->d_list};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (h->m) gempic_maxwell2d_destroy(h->m);
@@ -1019,6 +1199,8 @@ int gempic_splitting2d_set_particles(gempic_splitting2d *h, const double *aos, i
     hipLaunchKernelGGL(k_s2_in, dim3(gb), dim3(256), 0, h->stream, (const double *)h->d_stage, (int64_t)6, n, pm);
     S2_TRY("2D3V upload", hipGetLastError());
     h->steps_since_sort = 0;
+    h->binned = false;
+    h->f2_slow = false;
     int rc = h->sort_interval > 0 ? s2_sort(h) : GEMPIC_OK;   // sorted on upload where sorting is on
     if (rc) return rc;
     return s2_finish(h);
@@ -1119,7 +1301,40 @@ int gempic_splitting2d_strang_splitting(gempic_splitting2d *h, double dt, int64_
     if (n_steps < 0) return abi_fail(GEMPIC_ERR_ARGUMENT, "ArgumentError: number_steps must be >= 0");
     const double hdt = 0.5 * dt;
     int rc = GEMPIC_OK;
-    for (int64_t s = 0; s < n_steps && !rc; ++s) {
+    const bool fused = h->f2 && !h->f2_slow && h->n > 0;
+    if (fused && n_steps > 0) {
+        // HB and HE's B update of the first step; then per step one particle
+        // pass and the field work up to the next step's. E after the
+        // currents is the last HE's field of this step, es = that plus E
+        // after both HB the field of the two HE of a step's end and the
+        // next's begin.
+        s2_hb(h, hdt);
+        m2d_b_from_e(h->m, hdt, h->d_e, h->d_b);
+        for (int64_t s = 0; s < n_steps && !rc; ++s) {
+            if (h->sort_interval > 0 && h->steps_since_sort >= h->sort_interval) {
+                rc = s2_sort(h);
+                h->binned = false;
+            }
+            if (!rc && h->f2_strips > 1 && (!h->binned || h->steps_since_bin >= kBinEvery)) rc = f2_bin(h);
+            double *const *e = s == 0 ? h->d_e : h->d_es;
+            if (s + 1 < n_steps) {
+                if (!rc) rc = f2_pass(h, F2_ALL, dt, e);
+                if (rc) break;
+                m2d_b_from_e(h->m, hdt, h->d_e, h->d_b);
+                m2d_e_from_b(h->m, 2.0 * hdt, h->d_b, h->d_e, h->d_es);
+                m2d_b_from_e(h->m, hdt, h->d_e, h->d_b);
+            } else {
+                if (!rc) rc = f2_pass(h, F2_FIRST, dt, e);
+                if (!rc) rc = f2_pass(h, F2_SECOND, dt, e);
+                if (!rc) rc = s2_he(h, hdt);
+                if (!rc) rc = s2_hb(h, hdt);
+            }
+            h->steps_since_sort++;
+            h->steps_since_bin++;
+            h->f2_steps++;
+        }
+    }
+    for (int64_t s = 0; s < n_steps && !rc && !fused; ++s) {
         if (h->sort_interval > 0 && h->steps_since_sort >= h->sort_interval) rc = s2_sort(h);
         if (!rc) rc = s2_hb(h, hdt);
         if (!rc) rc = s2_he(h, hdt);

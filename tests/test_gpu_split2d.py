@@ -169,6 +169,35 @@ def test_gpu_2d3v_every_particle_once(n):
         _close(h.b_dofs[c], o_b[c], 1e-11, f"B{c + 1}")
 
 
+@pytest.mark.parametrize("degree, nx, ny, n, vscale, steps", [
+    (3, 48, 36, 5001, 0.8, 3),      # nine whole grids fill the LDS
+    (1, 9, 7, 777, 0.8, 3),         # the smallest passes
+    (3, 64, 64, 60001, 0.8, 12),    # strips, binned twice
+    (2, 100, 40, 30000, 0.8, 3),    # narrower strips, the last one short
+    (2, 40, 101, 3000, 0.3, 3),     # fewer particles than a workgroup's share
+    (3, 256, 16, 20000, 0.3, 2),    # no room for strips: the operators' passes
+    (3, 64, 64, 20000, 6.0, 2),     # paths across many cells and strips: all listed
+])
+def test_gpu_2d3v_fused_steps_match_oracle(degree, nx, ny, n, vscale, steps):
+    """strang_splitting's one-pass step against the oracle's operators: E, B,
+    the particles and the currents of the last step's operators. Rounding
+    alone differs (measured up to 3e-14 of each largest value); a second call
+    goes on from the first one's state."""
+    print(f"2d3v fused: degree {degree}, {nx} x {ny}, n={n}, v {vscale}, {steps} steps", flush=True)
+    w = _hot(n=n, nx=nx, ny=ny, L1=0.25 * nx, L2=0.25 * ny, seed=8, vscale=vscale, fscale=0.05)
+    h, pg, osp, o_parts, o_e, o_b = _pair(w, degree, sync=False)
+    for k in (steps, 1):
+        h.strang_splitting(0.05, k)
+        osp.strang_splitting(0.05, k)
+        h.to_host()
+        for r in range(5):
+            _close(pg.array[r], o_parts[r], 1e-11, f"row {r}")
+        for c in range(3):
+            _close(h.e_dofs[c], o_e[c], 1e-11, f"E{c + 1}")
+            _close(h.b_dofs[c], o_b[c], 1e-11, f"B{c + 1}")
+            _close(h.j_dofs[c], osp.j(c + 1), 1e-11, f"j{c + 1}")
+
+
 def test_gpu_2d3v_errors_and_order():
     w = _hot(n=1000)
     h, pg, *_ = _pair(w, 3)
@@ -177,6 +206,8 @@ def test_gpu_2d3v_errors_and_order():
     pg.array[0, 17] = float("nan")
     with pytest.raises(G.InexactError):
         h.operatorHE(0.1)
+    with pytest.raises(G.InexactError):
+        h.strang_splitting(0.1, 2)
     with pytest.raises(ValueError):
         mesh = G.TwoDGrid(0.0, 1.0, 128, 0.0, 1.0, 64)
         pg2 = G.ParticleGroup(2, 3, 10)
