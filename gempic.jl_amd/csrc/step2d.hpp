@@ -390,7 +390,7 @@ __global__ void __launch_bounds__(f2_threads(P)) k_step2d(F2Args a)
         };
         auto take_y = [&] {
             x2 = a.ymin + jl_mod(pn - a.ymin, a.Ly);
-            cy = ce;
+            cy = imod(ce, ny);          // as of the position after the mod
             r = re;
 #pragma unroll
             for (int k = 0; k <= P; ++k) by0[k] = ey0[k];
