@@ -18,6 +18,7 @@
 #include "../../include/gempic_hip.h"
 #include "host_setup.hpp"
 #include "lib_internal.hpp"
+#include "transfer.hpp"
 
 using namespace gl;
 
@@ -69,6 +70,12 @@ int device_cus()
 int gl::abi_fail(int code, const char *msg) { return fail(code, msg); }
 int gl::abi_check_device() { return check_device(); }
 int gl::abi_device_cus() { return device_cus(); }
+hipError_t gl::to_host(void *dst, const void *src, size_t bytes, hipStream_t after, int device)
+{
+    return TransferPool::get().to_host(dst, src, bytes, after, device);
+}
+void gl::transfer_acquire() { TransferPool::get().acquire(); }
+void gl::transfer_release() { TransferPool::get().release(); }
 
 namespace {
 
@@ -540,6 +547,7 @@ int gempic_splitting_create(int64_t nx, double xmin, double xmax, int maxwell_de
     if (rc) return rc;
 
     gempic_splitting *h = new gempic_splitting();
+    transfer_acquire();
     (void)hipGetDevice(&h->device);
     h->dim_v = dim_v;
     h->n_weights = n_weights;
@@ -565,6 +573,7 @@ int gempic_splitting_create(int64_t nx, double xmin, double xmax, int maxwell_de
     h->qm = charge / mass;
     gh::gauss_legendre((degree1 + 2) / 2, h->qx1, h->qw1);
     if (!gh::maxwell1d_tables(nx, maxwell_degree, h->tabs)) {
+        transfer_release();
         delete h;
         return fail(GEMPIC_ERR_ARGUMENT, "ArgumentError: invalid Maxwell1DFEM size");
     }
@@ -632,6 +641,7 @@ int gempic_splitting_destroy(gempic_splitting *h)
     for (auto &p : h->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
     for (auto e : h->pool) (void)hipEventDestroy(e);
     if (h->stream) (void)hipStreamDestroy(h->stream);
+    transfer_release();
     delete h;
     return GEMPIC_OK;
 }
@@ -740,7 +750,7 @@ int gempic_get_particles(gempic_splitting *h, double *aos, int64_t ld, int64_t n
     int rc = ensure_stage(h);
     if (rc) return rc;
     HIP_TRY(launch_soa_to_aos(h->d_stage, ld, n, h->dim_v, h->d_x, h->d_v1, h->d_v2, h->d_w, h->d_id, h->stream));
-    HIP_TRY(hipMemcpyAsync(aos, h->d_stage, sizeof(double) * (size_t)n * ld, hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(to_host(aos, h->d_stage, sizeof(double) * (size_t)n * ld, h->stream, h->device));
     return finish(h);
 }
 
@@ -754,23 +764,34 @@ int gempic_set_fields(gempic_splitting *h, const double *e1, const double *e2, c
     return finish(h);
 }
 
+// `count` neighbouring grid slots from `slot` on, in one copy, then to the
+// caller's arrays (any of them may be NULL)
+static int get_slots(gempic_splitting *h, int slot, int count, double *const *out)
+{
+    double tmp[3 * kNxMax];
+    HIP_TRY(hipMemcpyAsync(tmp, h->d_grid + slot * h->nx, sizeof(double) * count * h->nx, hipMemcpyDeviceToHost,
+                           h->stream));
+    const int rc = finish(h);
+    if (rc == GEMPIC_ERR_DEVICE) return rc;
+    for (int k = 0; k < count; ++k)
+        if (out[k]) std::memcpy(out[k], tmp + k * h->nx, sizeof(double) * h->nx);
+    return rc;
+}
+
 int gempic_get_fields(gempic_splitting *h, double *e1, double *e2, double *b)
 {
     CHECK_H(h);
-    const size_t nb = sizeof(double) * h->nx;
-    if (e1) HIP_TRY(hipMemcpyAsync(e1, h->d_grid + S_E1 * h->nx, nb, hipMemcpyDeviceToHost, h->stream));
-    if (e2) HIP_TRY(hipMemcpyAsync(e2, h->d_grid + S_E2 * h->nx, nb, hipMemcpyDeviceToHost, h->stream));
-    if (b) HIP_TRY(hipMemcpyAsync(b, h->d_grid + S_B * h->nx, nb, hipMemcpyDeviceToHost, h->stream));
-    return finish(h);
+    static_assert(S_E2 == S_E1 + 1 && S_B == S_E1 + 2, "neighbouring slots");
+    double *const out[3] = {e1, e2, b};
+    return get_slots(h, S_E1, 3, out);
 }
 
 int gempic_get_j(gempic_splitting *h, double *j1, double *j2)
 {
     CHECK_H(h);
-    const size_t nb = sizeof(double) * h->nx;
-    if (j1) HIP_TRY(hipMemcpyAsync(j1, h->d_grid + S_J1 * h->nx, nb, hipMemcpyDeviceToHost, h->stream));
-    if (j2) HIP_TRY(hipMemcpyAsync(j2, h->d_grid + S_J2 * h->nx, nb, hipMemcpyDeviceToHost, h->stream));
-    return finish(h);
+    static_assert(S_J2 == S_J1 + 1, "neighbouring slots");
+    double *const out[2] = {j1, j2};
+    return get_slots(h, S_J1, 2, out);
 }
 
 // the mode bit of the handle's arithmetic for its 1d2v particle passes
@@ -1187,8 +1208,7 @@ int gempic_get_adjoint(gempic_splitting *h, double *loss, double *g_particles, i
         // the cotangents are in the particle order the call started from
         HIP_TRY(launch_adj_rows_out(h->d_stage, ld, n, h->adj_id0, h->d_lam, h->d_lam + n,
                                     h->d_lam + 2 * n, h->stream));
-        HIP_TRY(hipMemcpyAsync(g_particles, h->d_stage, sizeof(double) * (size_t)n * ld,
-                               hipMemcpyDeviceToHost, h->stream));
+        HIP_TRY(to_host(g_particles, h->d_stage, sizeof(double) * (size_t)n * ld, h->stream, h->device));
     }
     if (g_e1) HIP_TRY(hipMemcpyAsync(g_e1, h->d_agrid + A_E1 * nx, fb, hipMemcpyDeviceToHost, h->stream));
     if (g_e2) HIP_TRY(hipMemcpyAsync(g_e2, h->d_agrid + A_E2 * nx, fb, hipMemcpyDeviceToHost, h->stream));

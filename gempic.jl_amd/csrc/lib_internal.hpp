@@ -292,6 +292,11 @@ hipError_t launch_pmc(int op, const PmcArgs &a, int blocks, hipStream_t s);
 int abi_fail(int code, const char *msg);
 int abi_check_device();
 int abi_device_cus();
+// a copy of GPU memory to the caller's array once the stream's work is done
+// (transfer.hpp); every handle that uses it counts as one user of its buffers
+hipError_t to_host(void *dst, const void *src, size_t bytes, hipStream_t after, int device);
+void transfer_acquire();
+void transfer_release();
 
 }  // namespace gl
 

@@ -676,6 +676,7 @@ __global__ void k_s2_out(double *aos, int64_t ld, int64_t n, S2Perm pm)
 struct gempic_splitting2d {
     gempic_maxwell2d *m = nullptr;
     hipStream_t stream = nullptr;           // the solver's stream
+    int device = 0;
     int nx = 0, ny = 0, p = 3;
     int64_t n = 0;
     double xmin = 0, ymin = 0, Lx = 0, Ly = 0, dx = 0, dy = 0;
@@ -1079,6 +1080,8 @@ int gempic_splitting2d_create(int64_t nx, int64_t ny, double xmin, double xmax, 
     rc = gempic_maxwell2d_create(nx, xmin, xmax, ny, ymin, ymax, degree, &m);
     if (rc) return rc;
     gempic_splitting2d *h = new gempic_splitting2d();
+    transfer_acquire();
+    (void)hipGetDevice(&h->device);
     h->m = m;
     h->stream = m2d_stream(m);
     h->nx = (int)nx;
@@ -1178,6 +1181,7 @@ int gempic_splitting2d_destroy(gempic_splitting2d *h)
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (h->m) gempic_maxwell2d_destroy(h->m);
+    transfer_release();
     delete h;
     return GEMPIC_OK;
 }
@@ -1220,8 +1224,7 @@ int gempic_splitting2d_get_particles(gempic_splitting2d *h, double *aos, int64_t
     const unsigned gb = (unsigned)std::max<int64_t>(1, std::min<int64_t>(4096, (n + 255) / 256));
     hipLaunchKernelGGL(k_s2_out, dim3(gb), dim3(256), 0, h->stream, h->d_stage, (int64_t)6, n, pm);
     S2_TRY("2D3V download", hipGetLastError());
-    S2_TRY("2D3V download", hipMemcpyAsync(aos, h->d_stage, sizeof(double) * 6 * (size_t)n,
-                                           hipMemcpyDeviceToHost, h->stream));
+    S2_TRY("2D3V download", to_host(aos, h->d_stage, sizeof(double) * 6 * (size_t)n, h->stream, h->device));
     return s2_finish(h);
 }
 

@@ -409,3 +409,24 @@ def test_gpu_save_and_resume(tmp_path):
     assert_rows_close(pgc.array, pga.array, 1e-11)
     for got, ref in ((c.e_dofs[0], a.e_dofs[0]), (c.e_dofs[1], a.e_dofs[1]), (c.b_dofs, a.b_dofs)):
         assert np.max(np.abs(got - ref)) <= 1e-11 * max(np.max(np.abs(ref)), 1.0)
+
+
+@pytest.mark.parametrize("n", [131071, 131072, 131073, 700001])
+def test_gpu_particles_come_back_whole(n):
+    """Downloads around the size from which several threads copy chunks (4 MiB:
+    131,072 particles), a last chunk that is not full, and two handles read
+    from two threads at once: the uploaded particles, bit for bit."""
+    import threading
+    print(f"particle round trip, n={n}", flush=True)
+    pairs = [_setup_pair(_hot_weibel(n, seed=s)) for s in (1, 2)]
+    want = [pg.array.copy() for _, pg, *_ in pairs]
+    for h, pg, *_ in pairs:
+        h.to_device()
+        pg.array[:] = 0.0
+    threads = [threading.Thread(target=h.to_host) for h, *_ in pairs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for w, (_, pg, *_) in zip(want, pairs):
+        np.testing.assert_array_equal(pg.array, w)
