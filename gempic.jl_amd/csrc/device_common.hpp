@@ -347,6 +347,32 @@ __device__ __forceinline__ double lane_value(double v, int l)
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
+// Within quads of lanes (all active): the value of the quad's lane T in each
+// of its lanes, and the transpose of a 4 x 4 matrix held one row per lane.
+template <int T>
+__device__ __forceinline__ double quad_lane(double v) { return dpp_f64<T * 0x55>(v); }
+template <int T>
+__device__ __forceinline__ int quad_lane(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, T * 0x55, 0xf, 0xf, true);
+}
+__device__ __forceinline__ void quad_transpose(double (&c)[4])
+{
+    const bool odd = threadIdx.x & 1, high = threadIdx.x & 2;
+#pragma unroll
+    for (int k = 0; k < 4; k += 2) {
+        const double r = dpp_f64<0xB1>(odd ? c[k] : c[k + 1]);       // quad_perm [1, 0, 3, 2]
+        c[k] = odd ? r : c[k];
+        c[k + 1] = odd ? c[k + 1] : r;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const double r = dpp_f64<0x4E>(high ? c[k] : c[k + 2]);      // quad_perm [2, 3, 0, 1]
+        c[k] = high ? r : c[k];
+        c[k + 2] = high ? c[k + 2] : r;
+    }
+}
+
 // row[node] += the wave's sums of v[w], node = first_node(cell, W-1) + w: one
 // LDS add by the first lane of each row of 16 that holds a sum. Only this
 // wave adds to its row and its LDS operations run in order, so the order of

@@ -18,6 +18,7 @@
 #include <cmath>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/gempic_hip.h"
@@ -51,7 +52,7 @@ constexpr int kGrid2Max = 4096;            // nx*ny of the device deposit (LDS g
 #define GEMPIC_DEP_WAVES 4
 #endif
 #ifndef GEMPIC_DEP_WAVES_FAST
-#define GEMPIC_DEP_WAVES_FAST 4
+#define GEMPIC_DEP_WAVES_FAST 8
 #endif
 #ifndef GEMPIC_DEP_BLOCKS_PER_CU
 #define GEMPIC_DEP_BLOCKS_PER_CU 0
@@ -77,7 +78,8 @@ struct Pmc2Args {
 
 // compute_shape_factor (particle_mesh_coupling_2d.jl:54-65): ceil() index, offset (0, 1]; returns the
 // first node (sx, sy) of the (P+1)^2 patch, wrapped into the grid
-template <int P>
+// (with FAST the splines' closed forms, equal to rounding, not bitwise)
+template <int P, bool FAST = false>
 __device__ __forceinline__ bool shape2(const Pmc2Args &a, double x, double y, int &sx, int &sy,
                                        double (&vx)[P + 1], double (&vy)[P + 1])
 {
@@ -86,8 +88,14 @@ __device__ __forceinline__ bool shape2(const Pmc2Args &a, double x, double y, in
     const bool ok = fabs(xp) < 1.0e9 && fabs(yp) < 1.0e9;
     const double cx = ok ? ceil(xp) : 0.0, cy = ok ? ceil(yp) : 0.0;
     const int ip = (int)cx, jp = (int)cy;
-    bspline<P>(ok ? xp - (double)(ip - 1) : 1.0, vx);
-    bspline<P>(ok ? yp - (double)(jp - 1) : 1.0, vy);
+    const double ox = ok ? xp - (cx - 1.0) : 1.0, oy = ok ? yp - (cy - 1.0) : 1.0;
+    if constexpr (FAST) {
+        bspline_fast<P>(ox, vx);
+        bspline_fast<P>(oy, vy);
+    } else {
+        bspline<P>(ox, vx);
+        bspline<P>(oy, vy);
+    }
     // index_1dto2d_column_major (:76-82): nodes ip - P - 1 + a, mod n
     sx = imod(ip - P - 1, a.nx);
     sy = imod(jp - P - 1, a.ny);
@@ -126,21 +134,18 @@ __device__ __forceinline__ bool shape2_pp(const Pmc2Args &a, double x, double y,
     return ok;
 }
 
-// Deposit (add_charge!, :94-105). Each lane keeps the (P+1)^2 node sums of
+// add_charge! (:94-105) in the deterministic mode. Each lane keeps the (P+1)^2 node sums of
 // the patch its particles fall in, in registers; when its next particle
 // starts another patch, the cached sums are flushed into an LDS grid:
 //  * if every flushing lane of the wave holds the same patch (particles
 //    sorted by cell), the wave sums them (DPP, fixed order) and 16 lanes add
 //    the patch to the grid;
-//  * otherwise, in the fast mode (DET = false), each flushing lane adds its
-//    patch with LDS atomics into the workgroup's shared grid;
-//  * in the deterministic mode (DET = true) every wave owns its grid and the
-//    flushing lanes add in passes: per pass, the lowest lane of each hash
-//    slot of its patch adds its whole patch (distinct patches, so no two
-//    lanes of one instruction hit one node), in lane order of the slots.
-// In the deterministic mode every addition's order is a fixed function of
+//  * otherwise the flushing lanes add in passes: per pass, the lowest lane of
+//    each hash slot of its patch adds its whole patch (distinct patches, so no
+//    two lanes of one instruction hit one node), in lane order of the slots.
+// Every wave owns its grid, so every addition's order is a fixed function of
 // the particle order; the waves' grids are summed in wave order at the end.
-template <int P, bool DET, bool PP>
+template <int P, bool PP>
 __global__ void __launch_bounds__(1024) k_pmc2d_deposit(Pmc2Args a)
 {
     constexpr int W = P + 1, WW = W * W;
@@ -149,8 +154,8 @@ __global__ void __launch_bounds__(1024) k_pmc2d_deposit(Pmc2Args a)
     const int nn = a.nx * a.ny;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int nw = blockDim.x / kWave;
-    const int ngrids = DET ? nw : 1;
-    double *grid = smem + (DET ? (size_t)wave * nn : 0);
+    const int ngrids = nw;
+    double *grid = smem + (size_t)wave * nn;
     double *stage = smem + (size_t)ngrids * nn + wave * 16;
     int *hash = (int *)(smem + (size_t)ngrids * nn + nw * 16) + wave * 256;
     for (int k = threadIdx.x; k < ngrids * nn; k += blockDim.x) smem[k] = 0.0;
@@ -183,11 +188,6 @@ __global__ void __launch_bounds__(1024) k_pmc2d_deposit(Pmc2Args a)
                 if (lane == kWave - 1) stage[j] = sj;
             }
             if (lane < WW) atomicAdd(&grid[node(k0, lane)], stage[lane]);
-        } else if constexpr (!DET) {
-            if (evict) {
-#pragma unroll
-                for (int j = 0; j < WW; ++j) atomicAdd(&grid[node(ckey, j)], acc[j]);
-            }
         } else {
             bool rem = evict;
             while (__ballot(rem)) {
@@ -255,6 +255,181 @@ __global__ void __launch_bounds__(1024) k_pmc2d_deposit(Pmc2Args a)
     }
 }
 
+constexpr int kFlushPatches = 4, kFlushShared = 8;
+
+// Row stride of a deposit grid with halo (nx + P columns), congruent to 4
+// modulo 16 doubles: the 16 nodes of a 4 x 4 patch fall in 16 different pairs
+// of banks.
+__host__ __device__ __forceinline__ int halo_stride(int nx, int p)
+{
+    return nx + p + ((20 - (nx + p) % 16) % 16);
+}
+
+// add_charge! in the fast mode. The workgroup's LDS grid has a halo of P
+// columns and rows, so that a patch is constant offsets from its first node.
+// A wave deposits in one of two ways, by the order its particles come in:
+//  * directly, every particle's patch with LDS atomics (particles in no order).
+//    Bound by the atomics: 64 lanes at random nodes take 18 cycles, as several
+//    meet in a bank. So the lanes of a quad take one column each of the same
+//    particle's patch (the quad's four particles in turn): 4 neighbouring nodes
+//    hit 4 neighbouring banks, and fewer collide;
+//  * through the lane's cached patch (particles sorted by cell), flushed when
+//    its next particle starts another one
+//    (patches that 8 of them hold: one DPP sum each).
+// It goes over to the first when half of the wave's lanes start another patch
+// at once, to the second when three quarters stay in theirs or a quarter of
+// them meet in one patch. us for 16,777,216 particles on 64 x 64, degree 3, in
+// no order and sorted by cell: 242 and 129 with every deposit through the
+// cache and 4 waves a workgroup, 200 and 125 (8 waves; 4: 205 and 131;
+// without the quads 213 and 111); 300,000 at degree 2: 23.1 and 27.9, 19.5
+// and 21.2. The bytes' time at a copy's rate is 83.
+template <int P, bool PP>
+__global__ void __launch_bounds__(kWave *GEMPIC_DEP_WAVES_FAST) k_pmc2d_deposit_fast(Pmc2Args a)
+{
+    constexpr int W = P + 1, WW = W * W;
+    extern __shared__ double smem[];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int nw = blockDim.x / kWave;
+    const int S = halo_stride(a.nx, P), gsz = S * (a.ny + P);
+    for (int k = threadIdx.x; k < gsz; k += blockDim.x) smem[k] = 0.0;
+    __syncthreads();
+    double *grid = smem;
+
+    int errs = 0;
+    const int64_t wbase = ((int64_t)blockIdx.x * nw + wave) * a.chunk;
+    const int64_t wend = wbase + a.chunk < a.n ? wbase + a.chunk : a.n;
+    // the next particle's inputs are loaded while the current one is deposited
+    int64_t i = wbase + lane;
+    double xn = 0.0, yn = 0.0, wn = 0.0;
+    auto load = [&] {
+        const int64_t k = i < wend ? i : wbase;
+        xn = a.x[k];
+        yn = a.y[k];
+        wn = a.w[k];
+    };
+    if (wbase < wend) load();
+    bool valid = false;
+    int o = 0;                      // the particle's first node
+    double ws = 0.0, vx[W], vy[W];
+    auto next = [&] {
+        const double x = xn, y = yn;
+        valid = i < wend;
+        ws = valid ? wn * a.scaling : 0.0;      // a lane without a particle adds zeros
+        i += kWave;
+        load();
+        int sx = 0, sy = 0;
+        const bool ok = PP ? shape2_pp<P>(a, x, y, sx, sy, vx, vy) : shape2<P, true>(a, x, y, sx, sy, vx, vy);
+        if (valid && !ok) errs |= E_INEXACT;
+        o = sx + sy * S;
+    };
+
+    int base = -1;                  // the first node of the lane's last particle
+    bool more = wbase < wend;
+    if (more) next();
+    while (more) {
+        // directly, until three quarters of the lanes stay in their patch or a
+        // quarter of them meet in one
+        for (;;) {
+            if (__popcll(__ballot(o == __builtin_amdgcn_readfirstlane(o))) > kWave / 4) {
+                base = -1;
+                break;
+            }
+            if constexpr (P == 3) {
+                quad_transpose(vx);
+                auto turn = [&](auto t) {
+                    constexpr int T = decltype(t)::value;
+                    const int node = quad_lane<T>(o) + (lane & 3);
+#pragma unroll
+                    for (int ib = 0; ib < W; ++ib)
+                        unsafeAtomicAdd(&grid[node + ib * S], vx[T] * quad_lane<T>(ws * vy[ib]));
+                };
+                turn(std::integral_constant<int, 0>{});
+                turn(std::integral_constant<int, 1>{});
+                turn(std::integral_constant<int, 2>{});
+                turn(std::integral_constant<int, 3>{});
+            } else {
+#pragma unroll
+                for (int ia = 0; ia < W; ++ia)
+#pragma unroll
+                    for (int ib = 0; ib < W; ++ib)
+                        unsafeAtomicAdd(&grid[o + ia + ib * S], (ws * vx[ia]) * vy[ib]);
+            }
+            base = o;
+            more = i - lane < wend;
+            if (!more) break;
+            next();
+            if (__popcll(__ballot(valid && o != base)) <= kWave / 4) break;
+        }
+        if (!more) break;
+        // through the lane's patch, until half of the lanes leave theirs
+        double acc[WW];
+#pragma unroll
+        for (int j = 0; j < WW; ++j) acc[j] = 0.0;
+        auto flush = [&](bool evict) {
+            evict = evict && base >= 0;
+            // a patch that several lanes hold: one sum over them (for the first
+            // few patches; same-node atomics of one instruction serialize)
+            unsigned long long m = __ballot(evict);
+            bool rest = evict;
+            for (int r = 0; r < kFlushPatches && m; ++r) {
+                const int k0 = __builtin_amdgcn_readlane(base, __builtin_ctzll(m));
+                const bool mine = rest && base == k0;
+                const unsigned long long mk = __ballot(mine);
+                m &= ~mk;
+                if (__popcll(mk) < kFlushShared) continue;
+#pragma unroll
+                for (int j0 = 0; j0 < WW; j0 += 4) {
+                    double q[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) q[u] = j0 + u < WW && mine ? acc[j0 + u < WW ? j0 + u : 0] : 0.0;
+                    const double s = wave_sum_quad<4>(q);
+                    const int j = j0 + quad_value(lane >> 4);
+                    if ((lane & 15) == 0 && j < WW) unsafeAtomicAdd(&grid[k0 + j / W + (j % W) * S], s);
+                }
+                rest = rest && !mine;
+            }
+            if (rest) {
+#pragma unroll
+                for (int j = 0; j < WW; ++j) unsafeAtomicAdd(&grid[base + j / W + (j % W) * S], acc[j]);
+            }
+            if (evict) {
+#pragma unroll
+                for (int j = 0; j < WW; ++j) acc[j] = 0.0;
+            }
+        };
+        for (;;) {
+            const bool leaves = valid && o != base;
+            if (__popcll(__ballot(leaves && base >= 0)) > kWave / 2) break;
+            flush(leaves);
+            if (valid) base = o;
+#pragma unroll
+            for (int ia = 0; ia < W; ++ia) {
+                const double wx = ws * vx[ia];
+#pragma unroll
+                for (int ib = 0; ib < W; ++ib) acc[ia * W + ib] = __builtin_fma(wx, vy[ib], acc[ia * W + ib]);
+            }
+            more = i - lane < wend;
+            if (!more) break;
+            next();
+        }
+        flush(true);
+    }
+    if (errs) atomicOr(a.err, errs);
+    __syncthreads();
+    double *out = a.part + (size_t)blockIdx.x * a.nx * a.ny;
+    for (int k = threadIdx.x; k < a.nx * a.ny; k += blockDim.x) {
+        const int gy = k / a.nx, gx = k - gy * a.nx;
+        const double *g = grid + gx + gy * S;
+        double t = g[0];
+        if (gx < P) t += g[a.nx];
+        if (gy < P) {
+            t += g[a.ny * S];
+            if (gx < P) t += g[a.ny * S + a.nx];
+        }
+        out[k] = t;
+    }
+}
+
 // sum of col[b * nn] for b in [b0, b1), added in order; the loads are issued
 // eight at a time
 __device__ __forceinline__ double sum_column(const double *col, int b0, int b1, int nn)
@@ -291,29 +466,30 @@ __global__ void k_pmc2d_reduce2(const double *part2, int splits, int nn, double 
 }
 
 // evaluate (:189-203) and evaluate_multiple (:214-231). With STAGE the
-// field is copied into LDS first: evaluate's with a periodic halo of P
-// columns and rows ((nx+P) x (ny+P), so the 16 reads of a particle are
-// constant offsets from its first node), evaluate_multiple's two fields
-// interleaved (one 16-byte read per node). The next particle's position is
-// loaded while the current one is evaluated.
+// field is copied into LDS first with a periodic halo of P columns and rows
+// ((nx+P) x (ny+P), so the 16 reads of a particle are constant offsets from
+// its first node), evaluate_multiple's two fields interleaved (one 16-byte
+// read per node). The next particle's position is loaded while the current
+// one is evaluated; loading two or four ahead ran slower (16,777,216
+// particles: 186 and 256 us against 172). evaluate_multiple took 184 us with
+// its fields staged without a halo; bound by VALU issue (the reference's
+// rounding: no fused multiply-adds), at 3.1 TB/s.
 template <int P, bool MULTI, bool STAGE>
 __global__ void __launch_bounds__(1024) k_pmc2d_eval(Pmc2Args a)
 {
     constexpr int W = P + 1;
     extern __shared__ __align__(16) double sfield[];
-    const int sw = STAGE && !MULTI ? a.nx + P : a.nx;       // row stride of the staged field
+    const int sw = STAGE ? a.nx + P : a.nx;                 // row stride of the staged field
     if constexpr (STAGE) {
-        if constexpr (MULTI) {
-            const int nn = a.nx * a.ny;
-            for (int k = threadIdx.x; k < nn; k += blockDim.x) {
-                sfield[2 * k] = a.f1[k];
-                sfield[2 * k + 1] = a.f2[k];
-            }
-        } else {
-            const int ns = sw * (a.ny + P);
-            for (int k = threadIdx.x; k < ns; k += blockDim.x) {
-                const int gy = k / sw, gx = k - gy * sw;
-                sfield[k] = a.f1[(gx < a.nx ? gx : gx - a.nx) + (gy < a.ny ? gy : gy - a.ny) * a.nx];
+        const int ns = sw * (a.ny + P);
+        for (int k = threadIdx.x; k < ns; k += blockDim.x) {
+            const int gy = k / sw, gx = k - gy * sw;
+            const int g = (gx < a.nx ? gx : gx - a.nx) + (gy < a.ny ? gy : gy - a.ny) * a.nx;
+            if constexpr (MULTI) {
+                sfield[2 * k] = a.f1[g];
+                sfield[2 * k + 1] = a.f2[g];
+            } else {
+                sfield[k] = a.f1[g];
             }
         }
         __syncthreads();
@@ -339,6 +515,17 @@ __global__ void __launch_bounds__(1024) k_pmc2d_eval(Pmc2Args a)
             for (int ia = 0; ia < W; ++ia)
 #pragma unroll
                 for (int ib = 0; ib < W; ++ib) v1 += f[ia + ib * sw] * vx[ia] * vy[ib];
+        } else if constexpr (STAGE) {
+            const double2 *f = f12 + sx + sy * sw;
+#pragma unroll
+            for (int ia = 0; ia < W; ++ia)
+#pragma unroll
+                for (int ib = 0; ib < W; ++ib) {
+                    const double c = vx[ia] * vy[ib];
+                    const double2 g = f[ia + ib * sw];
+                    v1 += g.x * c;
+                    v2 += g.y * c;
+                }
         } else {
             int gx = sx;
 #pragma unroll
@@ -349,17 +536,8 @@ __global__ void __launch_bounds__(1024) k_pmc2d_eval(Pmc2Args a)
                     const int k = gx + gy * a.nx;
                     if constexpr (MULTI) {
                         const double c = vx[ia] * vy[ib];
-                        double g1, g2;
-                        if constexpr (STAGE) {
-                            const double2 g = f12[k];
-                            g1 = g.x;
-                            g2 = g.y;
-                        } else {
-                            g1 = a.f1[k];
-                            g2 = a.f2[k];
-                        }
-                        v1 += g1 * c;
-                        v2 += g2 * c;
+                        v1 += a.f1[k] * c;
+                        v2 += a.f2[k] * c;
                     } else {
                         v1 += a.f1[k] * vx[ia] * vy[ib];
                     }
@@ -1487,7 +1665,11 @@ int ws2_get(size_t part_doubles, Ws2 *&w)
 }
 
 template <int P, bool DET, bool PP>
-const void *dep_fn() { return (const void *)k_pmc2d_deposit<P, DET, PP>; }
+const void *dep_fn()
+{
+    if constexpr (DET) return (const void *)k_pmc2d_deposit<P, PP>;
+    else return (const void *)k_pmc2d_deposit_fast<P, PP>;
+}
 
 template <bool PP>
 const void *dep_kernel_pp(int degree, bool det)
@@ -1501,12 +1683,12 @@ const void *dep_kernel(int degree, bool det, bool pp)
     return pp ? dep_kernel_pp<true>(degree, det) : dep_kernel_pp<false>(degree, det);
 }
 
-// LDS of k_pmc2d_deposit: grids (one per wave when deterministic), 16
-// staging doubles per wave, 256 hash slots per wave (deterministic)
-size_t dep_shmem(bool det, int nw, size_t nn)
+// LDS of k_pmc2d_deposit: a grid, 16 staging doubles and 256 hash slots per
+// wave; of k_pmc2d_deposit_fast: one grid with its halo (at most 41 KB)
+size_t dep_shmem(bool det, int nw, const Pmc2Args &a, int degree)
 {
-    return sizeof(double) * ((det ? (size_t)nw : 1) * nn + (size_t)nw * 16) +
-           (det ? sizeof(int) * 256 * (size_t)nw : 0);
+    if (!det) return sizeof(double) * (size_t)halo_stride(a.nx, degree) * (a.ny + degree);
+    return sizeof(double) * (size_t)nw * ((size_t)a.nx * a.ny + 16) + sizeof(int) * 256 * (size_t)nw;
 }
 
 struct DepPlan {
@@ -1516,20 +1698,20 @@ struct DepPlan {
 
 // waves per workgroup (4 unless the deterministic per-wave grids do not fit
 // in the workgroup's LDS) and workgroups (what the CUs hold at once)
-int dep_plan(int degree, bool det, bool pp, int64_t n, size_t nn, DepPlan &pl)
+int dep_plan(int degree, bool det, bool pp, const Pmc2Args &a, DepPlan &pl)
 {
     int dev = 0, maxsh = 65536, cus = abi_device_cus();
     if (hipGetDevice(&dev) == hipSuccess)
         (void)hipDeviceGetAttribute(&maxsh, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
     const void *fn = dep_kernel(degree, det, pp);
     int nw = det ? GEMPIC_DEP_WAVES : GEMPIC_DEP_WAVES_FAST;
-    while (nw > 1 && dep_shmem(det, nw, nn) > (size_t)maxsh) nw /= 2;
-    size_t sh = dep_shmem(det, nw, nn);
+    while (nw > 1 && dep_shmem(det, nw, a, degree) > (size_t)maxsh) nw /= 2;
+    size_t sh = dep_shmem(det, nw, a, degree);
     if (sh > 65536 &&
         hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh) != hipSuccess) {
         (void)hipGetLastError();
-        while (nw > 1 && dep_shmem(det, nw, nn) > 65536) nw /= 2;
-        sh = dep_shmem(det, nw, nn);
+        while (nw > 1 && dep_shmem(det, nw, a, degree) > 65536) nw /= 2;
+        sh = dep_shmem(det, nw, a, degree);
     }
     if (sh > (size_t)std::max(maxsh, 65536))
         return abi_fail(GEMPIC_ERR_ARGUMENT, "ArgumentError: the 2D grid does not fit in the deposit's LDS");
@@ -1539,7 +1721,7 @@ int dep_plan(int degree, bool det, bool pp, int64_t n, size_t nn, DepPlan &pl)
         occ = 1;
     }
     if (GEMPIC_DEP_BLOCKS_PER_CU > 0) occ = std::min(occ, GEMPIC_DEP_BLOCKS_PER_CU);
-    const int64_t want = (n + (int64_t)nw * kWave - 1) / ((int64_t)nw * kWave);
+    const int64_t want = (a.n + (int64_t)nw * kWave - 1) / ((int64_t)nw * kWave);
     pl.nw = nw;
     pl.sh = sh;
     pl.blocks = (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)cus * occ, want));
@@ -1558,7 +1740,7 @@ int pmc2_enqueue(int op, int degree, bool deterministic, Pmc2Args a, double *rho
     DepPlan pl;
     const bool charge = op == P2_CHARGE || op == P2_CHARGE_PP, pp = op == P2_CHARGE_PP;
     if (charge) {
-        int rc = dep_plan(degree, deterministic, pp, a.n, nn, pl);
+        int rc = dep_plan(degree, deterministic, pp, a, pl);
         if (rc) return rc;
         if (fixed) {
             const int64_t grids = (int64_t)(fixed->cap / nn);      // workgroup grids + split sums
@@ -1599,9 +1781,19 @@ int pmc2_enqueue(int op, int degree, bool deterministic, Pmc2Args a, double *rho
         else hipLaunchKernelGGL(k_pmc2d_eval_pp<3>, dim3(gb), dim3(256), 0, s, a);
     } else {
         const bool multi = op == P2_EVAL2;
-        const size_t ns = multi ? 2 * nn : (size_t)(a.nx + degree) * (a.ny + degree);
-        const bool stage = ns <= GEMPIC_EVAL_STAGE_MAX;                 // <= 64 KiB of LDS
+        // up to 64 KiB of LDS (two fields: of nodes; with their halo at most
+        // 83 KB, two workgroups to a CU all the same)
+        const size_t ns = (multi ? 2 : 1) * (size_t)(a.nx + degree) * (a.ny + degree);
+        const bool stage = (multi ? 2 * nn : ns) <= GEMPIC_EVAL_STAGE_MAX;
         const size_t sh = stage ? sizeof(double) * ns : 0;
+        if (sh > 65536) {
+            const void *fn = degree == 1 ? (const void *)k_pmc2d_eval<1, true, true>
+                             : degree == 2 ? (const void *)k_pmc2d_eval<2, true, true>
+                                           : (const void *)k_pmc2d_eval<3, true, true>;
+            const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
+            if (e != hipSuccess)
+                return abi_fail(GEMPIC_ERR_DEVICE, (std::string("2D evaluation: ") + hipGetErrorString(e)).c_str());
+        }
         const int nt = GEMPIC_EVAL_THREADS;
         const unsigned gb = (unsigned)std::max<int64_t>(
             1, std::min<int64_t>((int64_t)cus * GEMPIC_EVAL_BLOCKS_PER_CU, (a.n + nt - 1) / nt));

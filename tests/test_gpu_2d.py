@@ -397,6 +397,39 @@ def test_gpu_pmc2d_device_forms(degree):
     np.testing.assert_array_equal(o2.numpy(), r2)
 
 
+@pytest.mark.parametrize("degree, nx, ny, n", [(3, 256, 16, 300001), (3, 4, 256, 65), (2, 3, 3, 1000003),
+                                               (1, 64, 64, 1000003), (3, 64, 64, 1)])
+def test_gpu_pmc2d_deposit_in_mixed_orders(degree, nx, ny, n):
+    """The fast deposit changes between its two ways inside a wave's particles:
+    runs of one cell, of few cells and of no order, on the widest, the highest
+    and the smallest grids; evaluate_multiple's halo on the same grids."""
+    print(f"deposit orders: degree {degree}, {nx} x {ny}, n={n}", flush=True)
+    rng = np.random.default_rng(nx + ny)
+    bounds = (0.0, 3.0, -1.0, 1.0)
+    x, y = _particles(rng, n, bounds, nx, ny)
+    for k in range(0, n, 5000):                  # every other 5000 particles in one to three cells
+        if (k // 5000) % 2:
+            m = min(n, k + 5000)
+            c = rng.integers(0, 1 + (k // 5000) % 3, m - k)
+            x[k:m] = bounds[0] + (bounds[1] - bounds[0]) / nx * ((c % nx) + 0.1 + 0.8 * rng.random(m - k))
+            y[k:m] = bounds[2] + (bounds[3] - bounds[2]) / ny * (ny - 0.9 + 0.8 * rng.random(m - k))
+    w = rng.random(n)
+    _, pm = _coupling(nx, ny, bounds, degree, "galerkin", n)
+    p = orc.PMC2D(bounds[0], bounds[1], nx, bounds[2], bounds[3], ny, degree, orc.GALERKIN)
+    want = np.zeros(nx * ny)
+    _oracle_deposit(p, want, x, y, w)
+    D = DeviceArray.from_numpy
+    rho = DeviceArray.zeros(nx * ny)
+    G.add_charge_device_(rho, pm, D(x), D(y), D(w))
+    _assert_deposit(rho.numpy(), want)
+    f1, f2 = rng.normal(size=nx * ny), rng.normal(size=nx * ny)
+    o1, o2 = DeviceArray(n), DeviceArray(n)
+    G.evaluate_multiple_device(pm, (D(x), D(y)), (D(f1), D(f2)), (o1, o2))
+    r1, r2 = p.evaluate_multiple_n(x, y, f1, f2)
+    np.testing.assert_array_equal(o1.numpy(), r1)
+    np.testing.assert_array_equal(o2.numpy(), r2)
+
+
 def test_gpu_pmc2d_device_unstaged_eval_and_async_errors():
     rng = np.random.default_rng(33)
     nx, ny = 96, 80                    # 7680 nodes: two fields are read from global memory
