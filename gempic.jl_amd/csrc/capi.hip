@@ -376,6 +376,7 @@ int run_pass(gempic_splitting *h, int mode, double dt_he, double dt_hp2, double 
     a.chunk = L.chunk;
     a.iters = L.iters;
     a.ngroups = L.ngroups;
+    a.rgroups = epi_groups(L.blocks);
     set_generations(a, L, h->cus);
     a.dt_he = dt_he;
     a.dt_hp2 = dt_hp2;
@@ -389,12 +390,6 @@ int run_pass(gempic_splitting *h, int mode, double dt_he, double dt_hp2, double 
                                    pass_shmem_bytes((int)h->nx, mode), h->stream);
         if (e != hipSuccess)
             return fail(GEMPIC_ERR_DEVICE, std::string("particle pass launch: ") + hipGetErrorString(e));
-    }
-    if (mode_has_epi(mode)) {
-        ProfScope ps(h, 9);
-        hipError_t e = launch_epi(h->deg0, h->deg1, mode, a, L.blocks, h->stream);
-        if (e != hipSuccess)
-            return fail(GEMPIC_ERR_DEVICE, std::string("deposit sum launch: ") + hipGetErrorString(e));
     }
     return GEMPIC_OK;
 }

@@ -58,6 +58,7 @@ struct PassArgs {
     int iters;           // chunk / kBlock
     int nx;
     int ngroups;         // number of reduction groups
+    int rgroups;         // groups of the partial rows in the field part (epi_groups)
     int more;            // fused pass: another Strang step follows in this call
     int degree;          // write_step! degree argument (diagnostics)
     double xmin, dx, Lx;
@@ -73,7 +74,7 @@ struct PassArgs {
     unsigned *cnt;                // ngroups + 1 counters (zero between launches)
     int *err;                     // error flags
     double *diag;                 // diagnostics output (11 doubles)
-    double *hist;                 // fused Strang step with a record: k_epi1d writes B at the
+    double *hist;                 // fused Strang step with a record: the field part writes B at the
                                   // step's end to hist[4][nx] and the next pass's fields
                                   // E1, E2, B, E2P to hist[5..8][nx] (nullptr: no record)
     double *cx, *cv1, *cv2;       // fused Strang pass: also store x, v1, v2 here (nullptr: no)
@@ -109,11 +110,7 @@ hipError_t launch_pass_batch(int p0, int p1, int mode, const BatchArgs &b, int t
 hipError_t launch_epi_batch(int p0, int p1, int mode, const BatchArgs &b, int total_groups,
                             size_t shmem, hipStream_t s);
 size_t epi_shmem_bytes(int nx);
-int epi_groups(int nblocks);      // workgroups of the field part after a pass of nblocks
-// The deposit sum and field solves that follow a deposit pass (k_epi1d);
-// pass_blocks = workgroups of that pass. Modes with M_NOEPI have none.
-bool mode_has_epi(int mode);
-hipError_t launch_epi(int p0, int p1, int mode, const PassArgs &a, int pass_blocks, hipStream_t s);
+int epi_groups(int nblocks);      // groups of the partial rows of a pass of nblocks workgroups
 // workgroups of the (p0, p1, mode) pass kernel resident on one CU
 int pass_blocks_per_cu(int p0, int p1, int mode, size_t shmem);
 // LDS of a particle pass of this mode: padded fields, deposit rows (reused as
@@ -173,7 +170,7 @@ enum AdjRow { AR_E1 = 0, AR_E2, AR_B, AR_SCAL };   // AR_SCAL: [0] d/d dx, [1] d
 // scalars in the A_LOSS slot: the loss, then its explicit derivatives
 enum AdjScalar { AS_LOSS = 0, AS_DX, AS_MOD, AS_W };
 // field part of a reverse step: the reverse of the grid work between the
-// passes (k_epi1d and the prologue), see k_adj_epi
+// passes (epi1d_body and the prologue), see k_adj_epi
 enum AdjEpi : int { AE_TAIL = 0, AE_STEP, AE_HEAD, AE_POIS };
 // field record of one step (nx doubles each): the fields the step's pass
 // reads, then B at the step's end

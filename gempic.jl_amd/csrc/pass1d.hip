@@ -4,10 +4,10 @@
 // particle arrays once, with the fields of the pass in LDS, applies the
 // sub-steps selected by MODE to each particle in registers, and accumulates
 // the charge/current deposits with the deterministic per-lane cell caches of
-// device_common.hpp, writing one partial row per workgroup. The field part
-// (k_epi1d, a second launch) sums the rows in a fixed order (workgroup slices,
-// then the last of its workgroups to finish sums the group rows) and runs the
-// field solves of the sub-steps, so a whole Strang step is two launches.
+// device_common.hpp, writing one partial row per workgroup. The workgroups that
+// end last sum the rows in a fixed order (groups of rows, then the group rows)
+// and run the field solves of the sub-steps, so a whole Strang step is one
+// launch.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -470,11 +470,48 @@ __device__ __forceinline__ PassChunk pass_chunk(const PassArgs &a, int bid)
     return c;
 }
 
+// a partial row's entry, for the other workgroups of this launch (AGENT) or
+// for a later one
+template <bool AGENT>
+__device__ __forceinline__ void put_row(double *p, double v)
+{
+    if constexpr (AGENT) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *p = v;
+}
+template <bool AGENT>
+__device__ __forceinline__ double get_row(const double *p)
+{
+    if constexpr (AGENT) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else return *p;
+}
+
+// Count this workgroup in at *c once all its put_row<true> stores are done;
+// whether it is the last of n (the counter is then zero again for the next
+// launch). Called by all threads; `flag` is shared.
+__device__ __forceinline__ bool arrive_last(unsigned *c, unsigned n, int *flag)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const bool last =
+            __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+        if (last) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *flag = last;
+    }
+    __syncthreads();
+    return *flag != 0;
+}
+
+// the field part (below): PHASE 3 runs it at the end of the pass itself
+template <int P0, int P1, int MODE, int PHASE>
+__device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g, int ng, double *smem);
+
 // ---------------------------------------------------------------------------
-// The particle pass
+// The particle pass; with TAIL, the workgroup that ends last runs the field
+// part (nblocks workgroups in all)
 // ---------------------------------------------------------------------------
-template <int P0, int P1, int MODE>
-__device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *smem)
+template <int P0, int P1, int MODE, bool TAIL = false>
+__device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *smem, int nblocks = 0)
 {
     constexpr bool HE_PREV = (MODE & M_HE_PREV) != 0;
     constexpr bool HE = (MODE & M_HE) != 0;
@@ -806,9 +843,15 @@ __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *
             if (!((DEPMASK >> r) & 1u)) continue;
             double s = 0.0;
             for (int wv = 0; wv < kWaves; ++wv) s += rows[wv * len + idx];
-            a.part[(size_t)bid * len + idx] = s;
+            put_row<TAIL>(&a.part[(size_t)bid * len + idx], s);
         }
-        // the cross-workgroup sum and the field solves run in k_epi1d
+        // the cross-workgroup sum and the field solves (the sub-steps' are the
+        // same in either arithmetic)
+        if constexpr (TAIL) {
+            constexpr int STEP = M_HE | M_HP2A | M_HP1 | M_HP2B;
+            constexpr int EPI = (MODE & STEP) == STEP ? MODE : MODE & ~M_FAST;
+            epi1d_body<P0, P1, EPI, 3>(a, nblocks, bid, a.rgroups, smem);
+        }
     } else if constexpr (HE && !V1 && !HE_PREV) {
         // operatorHE alone: compute_b_from_e! after the push (:217-218). B is
         // not read by this pass, so workgroup 0 can update it at any time.
@@ -838,7 +881,8 @@ template <int P0, int P1, int MODE>
 __global__ void __launch_bounds__(kBlock, GEMPIC_PASS_MIN_WAVES) k_pass1d(PassArgs a)
 {
     extern __shared__ double smem[];
-    pass1d_body<P0, P1, MODE>(a, blockIdx.x, smem);
+    constexpr bool TAIL = (MODE & (M_HP2A | M_HP1 | M_HP2B | M_RHO)) != 0 && (MODE & M_NOEPI) == 0;
+    pass1d_body<P0, P1, MODE, TAIL>(a, blockIdx.x, smem, gridDim.x);
 }
 
 // One launch runs the same pass for every instance of an ensemble; each
@@ -856,14 +900,21 @@ __global__ void __launch_bounds__(kBlock) k_pass1d_batch(BatchArgs b)
 // The field part of a deposit pass: sum of the workgroups' partial rows and
 // the field solves of its sub-steps.
 //
-// It runs as a kernel of its own after the particle pass. The partial rows
-// are then visible to it through the kernel boundary, so the particle pass
-// needs no device-scope fence: on MI355X such a fence writes the XCD's whole
-// L2 back, and with the particle stores in flight hundreds of workgroups each
-// doing so cost more than the particle work. Here the L2 holds only this
-// kernel's few group rows, so its own fences are cheap: G workgroups each sum
-// a slice of the partial rows, and the last one to finish sums the G group
-// rows and runs the field solves.
+// It runs at the end of the particle pass, in the workgroup that ends last:
+// every workgroup stores its partial row, then counts itself in; the last of a
+// group of rows sums the group, the last of the groups sums the group rows and
+// runs the solves. A device-scope fence for the rows would write the XCD's
+// whole L2 back, particle stores and all (as a last-workgroup sum in the pass
+// it cost 81 us a step at 4,194,304 particles), so the rows are written and
+// read with agent-scope relaxed atomics, which go to the memory the XCDs share,
+// and a wave only waits for its own stores (s_waitcnt) before its workgroup
+// counts itself in. As a launch of its own the field part cost a dispatch
+// and its start on top (us per step, before and after): fused 1D2V 16,384
+// particles 15.2, 14.3; 300,001 25.7, 23.3; 1,048,576 31.7, 29.6; 4,194,304
+// 61.7, 59.1.
+//
+// The batched passes of an ensemble keep it in two launches (k_epi1d_batch):
+// there a workgroup's wait for its count would hold its place from the next.
 // ---------------------------------------------------------------------------
 
 // index r*nx + k of live entry e (the e-th entry of the rows in mask)
@@ -888,6 +939,7 @@ __device__ __forceinline__ int live_index(int e, int nx, unsigned mask)
 // sub-step passes' rows are summed in the same order at every row count; 1d1v
 // deposits one row and shares the threads over it (spread_rows = 1). Called
 // by all threads; scratch holds blockDim.x doubles.
+template <bool AGENT_IN, bool AGENT_OUT>
 __device__ void sum_rows(const double *base, int b0, int n, int stride, int nx, unsigned mask,
                          double *out, double *scratch, int spread_rows)
 {
@@ -911,7 +963,7 @@ __device__ void sum_rows(const double *base, int b0, int n, int stride, int nx, 
             for (int b = r0; b < r1; b += B) {      // a short last batch adds zeros
                 double t[B];
 #pragma unroll
-                for (int u = 0; u < B; ++u) t[u] = col[(size_t)(b + u < r1 ? b + u : r1 - 1) * rs];
+                for (int u = 0; u < B; ++u) t[u] = get_row<AGENT_IN>(&col[(size_t)(b + u < r1 ? b + u : r1 - 1) * rs]);
 #pragma unroll
                 for (int u = 0; u < B; ++u) s += b + u < r1 ? t[u] : 0.0;
             }
@@ -921,18 +973,19 @@ __device__ void sum_rows(const double *base, int b0, int n, int stride, int nx, 
         if (tid < ec) {
             double tot = 0.0;
             for (int hh = 0; hh < k; ++hh) tot += scratch[hh * ec + tid];
-            out[idx] = tot;
+            put_row<AGENT_OUT>(&out[idx], tot);
         }
         __syncthreads();
     }
 }
 
 // sum_rows over the rows [b0, b1)
+template <bool AGENT_IN = false, bool AGENT_OUT = false>
 __device__ __forceinline__ void sum_rows_range(const double *base, int b0, int b1, int nx,
                                                unsigned mask, double *out, double *scratch,
                                                int spread_rows = NDEP)
 {
-    sum_rows(base, b0, b1 - b0, 1, nx, mask, out, scratch, spread_rows);
+    sum_rows<AGENT_IN, AGENT_OUT>(base, b0, b1 - b0, 1, nx, mask, out, scratch, spread_rows);
 }
 
 // The first level of the field part's sum: group g of ng sums the partial
@@ -999,9 +1052,9 @@ __device__ __forceinline__ double circ_apply_t(const double *c, const double *rh
     return quad_sum(s);
 }
 
-// Workgroups of k_epi1d for nblocks partial rows: one while its threads hold
-// the rows in two batches of loads (no second level, fence or counter), else
-// the square root, which balances the two levels.
+// Groups of nblocks partial rows: one while its threads hold the rows in two
+// batches of loads (no second level), else the square root, which balances the
+// two levels.
 constexpr int kEpiOneGroup = 64;
 int epi_groups(int nblocks)
 {
@@ -1010,12 +1063,11 @@ int epi_groups(int nblocks)
     return g < 1 ? 1 : (g > kEpiGroupsMax ? kEpiGroupsMax : g);
 }
 
-// PHASE 0: the whole field part (the slice sums, then the last workgroup
-// to finish sums the group rows and runs the solves); PHASE 1: only this
-// workgroup's slice sum into its group row; PHASE 2: only the part after the
-// slice sums (a later launch, so no fences or counters are needed). Phases 1
-// and 2 together add the same numbers in the same order as phase 0.
-template <int P0, int P1, int MODE, int PHASE = 0>
+// PHASE 1: only workgroup g's sum of its group of rows into its group row;
+// PHASE 2: only the part after those sums (a later launch); PHASE 3: both, by
+// the pass's own workgroups (g: this one, of nblocks) as they end.
+// All add the same numbers in the same order.
+template <int P0, int P1, int MODE, int PHASE>
 __device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g, int ng,
                                            double *smem)
 {
@@ -1059,9 +1111,22 @@ __device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g
         return;
     }
 
-    // Every workgroup loads the fields and the tables it uses first (the one
-    // that ends up last then has them without another round trip), into
-    // registers, so that they arrive with the rows: nx <= kNxMax <= kBlock.
+    const double *last_rows = a.gpart;
+    int last_n = ng;
+    if constexpr (PHASE == 3) {
+        const int grp = ((g + 1) * ng - 1) / nblocks;          // the group with row g
+        const int b0 = (int)(((long)nblocks * grp) / ng), b1 = (int)(((long)nblocks * (grp + 1)) / ng);
+        if (!arrive_last(&a.cnt[1 + grp], (unsigned)(b1 - b0), &s_last)) return;
+        if (ng > 1) {
+            sum_rows_range<true, true>(a.part, b0, b1, nx, REDMASK, a.gpart + (size_t)grp * len, scratch, SPREAD);
+            if (!arrive_last(&a.cnt[0], (unsigned)ng, &s_last)) return;
+        } else {
+            last_rows = a.part;
+            last_n = nblocks;
+        }
+    }
+    // The fields and the tables used are loaded into registers, so that they
+    // arrive with the rows: nx <= kNxMax <= kBlock.
     static_assert(kNxMax <= kBlock, "one node per thread");
     constexpr int T0 = FAST ? T_CM0 : T_COS, TN = FAST ? 3 : 6;      // T_CM0..T_CAMP / T_COS..T_POIS
     static_assert(T_CAMP == T_CM0 + 2 && T_POIS == T_COS + 5, "contiguous tables");
@@ -1075,40 +1140,16 @@ __device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g
         for (int k = 0; k < TN; ++k) f_t[k] = a.tabs[(T0 + k) * nx + tid];
     }
     for (int i = tid; i < len; i += nt) sRed[i] = 0.0;
-    auto stage = [&] {
-        if (tid < nx) {
-            sE1[tid] = f_e1;
-            sE2[tid] = f_e2;
-            sB[tid] = f_b;
+    __syncthreads();
+    sum_rows_range<PHASE == 3, false>(last_rows, 0, last_n, nx, REDMASK, sRed, scratch, SPREAD);
+    if (tid < nx) {
+        sE1[tid] = f_e1;
+        sE2[tid] = f_e2;
+        sB[tid] = f_b;
 #pragma unroll
-            for (int k = 0; k < TN; ++k) T[(T0 + k) * nx + tid] = f_t[k];
-        }
-    };
-
-    if (PHASE == 0 && ng == 1) {
-        __syncthreads();                        // sRed is zero
-        sum_rows_range(a.part, 0, nblocks, nx, REDMASK, sRed, scratch, SPREAD);
-        stage();
-        __syncthreads();
-    } else {
-        if constexpr (PHASE == 0) {
-            // group sums of a slice of the workgroups' rows
-            sum_group_rows(a.part, nblocks, g, ng, nx, REDMASK, a.gpart + (size_t)g * len, scratch, SPREAD);
-            stage();
-            __threadfence();
-            __syncthreads();
-            if (tid == 0) s_last = atomicAdd(&a.cnt[0], 1u) == (unsigned)(ng - 1);
-            __syncthreads();
-            if (!s_last) return;
-            __threadfence();
-            if (tid == 0) a.cnt[0] = 0u;            // counters are zero between launches
-        } else {
-            (void)s_last;
-            stage();
-            __syncthreads();
-        }
-        sum_rows_range(a.gpart, 0, ng, nx, REDMASK, sRed, scratch, SPREAD);  // ends with a barrier
+        for (int k = 0; k < TN; ++k) T[(T0 + k) * nx + tid] = f_t[k];
     }
+    __syncthreads();
     double *r_j2a = sRed + D_J2A * nx, *r_j1 = sRed + D_J1 * nx;
     double *r_rho = sRed + D_RHO * nx, *r_j2b = sRed + D_J2B * nx;
     if constexpr (RHO_ONLY) {
@@ -1264,13 +1305,6 @@ __device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g
     }
 }
 
-template <int P0, int P1, int MODE>
-__global__ void __launch_bounds__(kBlock) k_epi1d(PassArgs a, int nblocks)
-{
-    extern __shared__ double smem[];
-    epi1d_body<P0, P1, MODE>(a, nblocks, blockIdx.x, gridDim.x, smem);
-}
-
 // The field parts of every instance of an ensemble in two launches: the
 // slice sums (instance i's epi_groups(its pass workgroups) workgroups are
 // [epi_start[i], epi_start[i+1])), then one workgroup per instance for the
@@ -1418,55 +1452,6 @@ __global__ void __launch_bounds__(kBlock) k_diag1d2v(PassArgs a)
 // ---------------------------------------------------------------------------
 // Launch dispatch
 // ---------------------------------------------------------------------------
-bool mode_has_epi(int m)
-{
-    return (m & (M_HP2A | M_HP1 | M_HP2B | M_RHO)) != 0 && (m & M_NOEPI) == 0;
-}
-
-template <int P0, int P1>
-static hipError_t launch_epi_pd(int mode, const PassArgs &a, int pass_blocks, hipStream_t s)
-{
-#define GK_EPI(M)                                                                             \
-    case (M):                                                                                 \
-        hipLaunchKernelGGL((k_epi1d<P0, P1, (M)>), dim3(epi_groups(pass_blocks)), dim3(kBlock), \
-                           epi_shmem_bytes(a.nx), s, a, pass_blocks);                         \
-        return hipGetLastError();
-    switch (mode) {
-        GK_EPI(M_HP2A)
-        GK_EPI(M_HP1)
-        GK_EPI(M_HE | M_HP2A | M_HP1 | M_HP2B)
-        GK_EPI(M_HE_PREV | M_HE | M_HP2A | M_HP1 | M_HP2B)
-        GK_EPI(M_FAST | M_HE | M_HP2A | M_HP1 | M_HP2B)
-        GK_EPI(M_FAST | M_HE_PREV | M_HE | M_HP2A | M_HP1 | M_HP2B)
-        GK_EPI(M_HP1 | M_HP2B | M_WITH_J2A)
-        GK_EPI(M_V1 | M_HP1)
-        GK_EPI(M_V1 | M_HE | M_HP1)
-        GK_EPI(M_V1 | M_HE_PREV | M_HE | M_HP1)
-        GK_EPI(M_RHO)
-    default:
-        return hipErrorInvalidValue;
-    }
-#undef GK_EPI
-}
-
-hipError_t launch_epi(int p0, int p1, int mode, const PassArgs &a, int pass_blocks, hipStream_t s)
-{
-    if (a.nx > kNxMax || pass_blocks < 1) return hipErrorInvalidValue;
-    // the sub-step modes' field parts are the same in either arithmetic
-    if ((mode & M_FAST) && (mode & (M_HE | M_HP2A | M_HP1 | M_HP2B)) != (M_HE | M_HP2A | M_HP1 | M_HP2B))
-        mode &= ~M_FAST;
-#define GK_PAIR(A, B) \
-    if (p0 == (A) && p1 == (B)) return launch_epi_pd<A, B>(mode, a, pass_blocks, s);
-    GK_PAIR(1, 0)
-    GK_PAIR(1, 1)
-    GK_PAIR(2, 1)
-    GK_PAIR(2, 2)
-    GK_PAIR(3, 2)
-    GK_PAIR(3, 3)
-#undef GK_PAIR
-    return hipErrorInvalidValue;
-}
-
 template <int P0, int P1>
 static hipError_t launch_batch_pd(bool epi, int mode, const BatchArgs &b, int total, size_t shmem,
                                   hipStream_t s)
@@ -1770,7 +1755,7 @@ __global__ void __launch_bounds__(kBlock) k_boris1d(PassArgs a)
 }
 
 // The field part after a Boris x push: the deposit sum over the workgroups'
-// rows (as k_epi1d: group slices, then the last workgroup), then
+// rows (group slices, then the last workgroup), then
 //  BE_J:       j_dofs = the deposits (push_x_accumulate_j!);
 //  BE_STAGGER: staggering! (:103-121) with h = a.dt_hp1: E_mid = E,
 //              j = h j, E1_mid -= M1^-1 j1/dx, E2_mid += h W(B),
@@ -1801,7 +1786,7 @@ __global__ void __launch_bounds__(kBlock) k_boris_epi(PassArgs a, int nblocks)
     double *scratch = w3 + 6 * nx;          // [blockDim.x]
     double *G = a.grid;
     const int se1 = KIND == BE_STAGGER ? S_E1 : S_E1M, se2 = KIND == BE_STAGGER ? S_E2 : S_E2M;
-    // loaded into registers first, so that they arrive with the rows (as k_epi1d)
+    // loaded into registers first, so that they arrive with the rows (as epi1d_body)
     constexpr int TN = 5;                   // T_COS .. T_AMP
     static_assert(T_AMP == T_COS + TN - 1, "contiguous tables");
     double f_e1 = 0.0, f_e2 = 0.0, f_b = 0.0, f_t[TN];
@@ -3169,7 +3154,7 @@ __device__ __forceinline__ void adj_epi_body(const AdjArgs &A, int nblocks, int 
     double *G = A.agrid;
 
     // loaded into registers first, so that they arrive with the rows (as
-    // k_epi1d): the cotangents, B at the step's end, E2 of the step's HE pair
+    // epi1d_body): the cotangents, B at the step's end, E2 of the step's HE pair
     // (into the slots of tables not used here) and the circulant columns
     static_assert(T_CPOIS == T_CM0 + 4, "contiguous tables");
     constexpr int TN = KIND == AE_POIS ? 0 : 4;
