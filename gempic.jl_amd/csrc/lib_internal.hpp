@@ -319,6 +319,6 @@ bool m2d_fused(const gempic_maxwell2d *m);
 // the same for all three components (m2d_fused grids): their split sums at
 // part2[split][component][node], scale[c] each
 void m2d_e_from_parts3(gempic_maxwell2d *m, const double *part2, int splits, const double *scale,
-                       double *const *j, double *const *e);
+                       double *stray, int *flags, double *const *j, double *const *e);
 void m2d_rho_from_e(gempic_maxwell2d *m, double *const *e, double *rho);
 }  // namespace gl

@@ -302,7 +302,7 @@ constexpr int kPad = 4;
 // The NF fields src(0), src(1), ... staged one behind the other at dst, each
 // nx + 2 kPad doubles, two loads of a thread in flight: one round trip to
 // memory for all of them (up to 512 doubles), where a copy per field waited
-// for each in turn (a workgroup's start took 6200 cycles, FIXME now).
+// for each in turn (a workgroup's start took 6200 cycles so).
 template <int NF, class Src>
 __device__ __forceinline__ void stage_padded(double *dst, int nx, Src src)
 {

@@ -850,6 +850,8 @@ struct FieldJ3 {
     const double *kx[3];
     double *jout[3];
     double *tmp[3];
+    double *stray;      // the listed particles' currents, added here and cleared
+    int *flags;         // F2Args::flags
 };
 
 __global__ void __launch_bounds__(kFieldThreads) k_fj_rows3(Field2 f, const double *part2, int splits, FieldJ3 a)
@@ -859,13 +861,18 @@ __global__ void __launch_bounds__(kFieldThreads) k_fj_rows3(Field2 f, const doub
     const int r0 = blockIdx.x * kFieldRows, rows = min(kFieldRows, f.ny - r0);
     double *jr = lds, *kk = lds + kFieldRows * nx;
     const double *kx = a.kx[c];
+    if (blockIdx.x == 0 && c == 0 && threadIdx.x == 0) {     // count the listed particles, empty the list
+        a.flags[1] += a.flags[2];
+        a.flags[2] = 0;
+    }
     for (int m = threadIdx.x; m < nx; m += blockDim.x) kk[m] = kx[m];
     for (int t = threadIdx.x; t < rows * nx; t += blockDim.x) {
         const int k = r0 * nx + t;
         double v = 0.0;
 #pragma unroll 16
         for (int sp = 0; sp < splits; ++sp) v += part2[((size_t)sp * 3 + c) * nn + k];
-        v = v * a.scale[c];
+        v = (v + a.stray[(size_t)c * nn + k]) * a.scale[c];
+        a.stray[(size_t)c * nn + k] = 0.0;
         a.jout[c][k] = v;
         jr[t] = v;
     }
@@ -1315,12 +1322,12 @@ bool gl::m2d_e_from_parts(gempic_maxwell2d *m, const double *part2, int splits, 
 }
 
 void gl::m2d_e_from_parts3(gempic_maxwell2d *m, const double *part2, int splits, const double *scale,
-                           double *const *j, double *const *e)
+                           double *stray, int *flags, double *const *j, double *const *e)
 {
     const Field2 f = m->f();
     const FieldTabs t = field_tabs(m);
     FieldJ3 a{{scale[0], scale[1], scale[2]}, {t.k1x, t.k0x, t.k0x}, {j[0], j[1], j[2]},
-              {m->buf(9), m->buf(10), m->buf(11)}};
+              {m->buf(9), m->buf(10), m->buf(11)}, stray, flags};
     hipLaunchKernelGGL(k_fj_rows3, dim3((m->ny + kFieldRows - 1) / kFieldRows, 3), dim3(kFieldThreads),
                        sizeof(double) * (size_t)(kFieldRows + 1) * m->nx, m->stream, f, part2, splits, a);
     FieldCols ca{{m->buf(9), m->buf(10), m->buf(11)}, {t.k0y, t.k1y, t.k0y}, {e[0], e[1], e[2]},

@@ -865,9 +865,12 @@ int s2_sort(gempic_splitting2d *h)
 // Steps between binnings by strip. Particles of the Landau configuration
 // drift 0.25 cells (rms) a step, 2.5 in ten, within the 5 rows to spare.
 constexpr int kBinEvery = 10;
-// The fused step's listed particles, of all in a step, from which the
-// operators' passes are the faster way: FIXME
-constexpr int kF2ListedMost = 32;
+// The fused step's listed particles a step from which the operators' passes
+// are the faster way. A listed particle costs 6.5 ns; the fused step saves
+// 100 us a step at 150,000 particles (71 against 175), 300 at 4,000,000 (404
+// against 710), 700 at 16,777,216: the ways meet at 14 % (measured; 11.5 % by
+// this rule), 1.2 % (1.0 %) and 0.6 % (0.7 %) listed.
+constexpr double f2_listed_most(int64_t n) { return 16384.0 + (double)n / 160.0; }
 
 int s2_finish(gempic_splitting2d *h)
 {
@@ -876,7 +879,7 @@ int s2_finish(gempic_splitting2d *h)
     S2_TRY("2D3V splitting", hipMemcpy(flags, h->d_err, sizeof(flags), hipMemcpyDeviceToHost));
     const int err = flags[0];
     if (h->f2_steps > 0) {
-        if ((double)flags[1] * kF2ListedMost > (double)h->n * (double)h->f2_steps) h->f2_slow = true;
+        if ((double)flags[1] > f2_listed_most(h->n) * (double)h->f2_steps) h->f2_slow = true;
         h->f2_steps = 0;
     }
     if (flags[0] || flags[1]) S2_TRY("2D3V splitting", hipMemset(h->d_err, 0, sizeof(flags)));
@@ -923,13 +926,13 @@ size_t f2_shmem(const gempic_splitting2d *h, int mode)
     return sizeof(double) * (size_t)((mode & F2_HE ? 9 : 6) * h->f2_s * h->f2_hr);
 }
 
-const void *f2_kernel(int p, int mode, bool listed = false)
+const void *f2_kernel(int p, int mode, bool rest = false)
 {
 #define F2K(P)                                                                                    \
-    if (listed)                                                                                   \
-        return mode == F2_ALL ? (const void *)k_f2_listed<P, F2_ALL>                              \
-               : mode == F2_FIRST ? (const void *)k_f2_listed<P, F2_FIRST>                        \
-                                  : (const void *)k_f2_listed<P, F2_SECOND>;                      \
+    if (rest)                                                                                     \
+        return mode == F2_ALL ? (const void *)k_f2_rest<P, F2_ALL>                                \
+               : mode == F2_FIRST ? (const void *)k_f2_rest<P, F2_FIRST>                          \
+                                  : (const void *)k_f2_rest<P, F2_SECOND>;                        \
     return mode == F2_ALL ? (const void *)k_step2d<P, F2_ALL>                                     \
            : mode == F2_FIRST ? (const void *)k_step2d<P, F2_FIRST>                               \
                               : (const void *)k_step2d<P, F2_SECOND>;
@@ -1018,15 +1021,14 @@ int f2_pass(gempic_splitting2d *h, int mode, double dt, double *const *e)
     void *args[] = {&a};
     S2_TRY("2D3V fused pass", hipLaunchKernel(f2_kernel(h->p, mode), dim3(nblk), dim3(nt), args,
                                               f2_shmem(h, mode), h->stream));
-    S2_TRY("2D3V listed particles", hipLaunchKernel(f2_kernel(h->p, mode, true), dim3(64), dim3(256), args, 0,
-                                                    h->stream));
     const int nn = h->nx * h->ny, splits = std::min(nblk, kSplits2);
     double *part2 = h->d_fpart + (size_t)h->blocks * 3 * h->f2_hr * h->nx;
-    hipLaunchKernelGGL(k_f2_reduce, dim3((unsigned)((nn + 255) / 256), (unsigned)splits, 3), dim3(256), 0, h->stream,
-                       a, h->p, nblk, part2);
-    S2_TRY("2D3V current sum", hipGetLastError());
+    void *rest[] = {&a, &nblk, &part2};
+    S2_TRY("2D3V listed particles and current sum",
+           hipLaunchKernel(f2_kernel(h->p, mode, true), dim3((unsigned)((nn + 255) / 256), (unsigned)splits, 4),
+                           dim3(256), rest, 0, h->stream));
     const double scale[3] = {1.0, 1.0, a.dt_half};
-    m2d_e_from_parts3(h->m, part2, splits, scale, h->d_j, h->d_e);
+    m2d_e_from_parts3(h->m, part2, splits, scale, a.stray, a.flags, h->d_j, h->d_e);
     return GEMPIC_OK;
 }
 

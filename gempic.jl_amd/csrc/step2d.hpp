@@ -52,7 +52,7 @@ struct F2Args {
     const double *w;
     const double *e[3], *b[3];
     double *part;                   // [workgroups][3][hr][nx] current sums
-    double *stray;                  // [3][nx * ny] currents of the listed particles
+    double *stray;                  // [3][nx * ny] currents of the listed particles; zero between steps
     int *list;                      // their indices (below 2^29), with the stage in the upper bits
     int *flags;                     // error bits, particles listed so far, in this pass
 };
@@ -223,18 +223,6 @@ __device__ __forceinline__ int f2_general(const F2Args &a, int64_t i, int stage)
     a.v2[i] = v2;
     a.v3[i] = v3;
     return errs;
-}
-
-template <int P, int MODE>
-__global__ void __launch_bounds__(256) k_f2_listed(F2Args a)
-{
-    const int n = a.flags[2];
-    int errs = 0;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
-        const int it = a.list[t];
-        errs |= f2_general<P, MODE>(a, it & 0x1fffffff, it >> 29);
-    }
-    if (errs) atomicOr(a.flags, errs);
 }
 
 template <int P, int MODE>
@@ -599,25 +587,37 @@ __global__ void __launch_bounds__(f2_threads(P)) k_step2d(F2Args a)
     }
 }
 
-// part2[split][component][node] = sum over the split's workgroups, in order,
-// of the rows they hold of the node's row; split 0 adds (and clears) the
-// listed particles' currents
-__global__ void __launch_bounds__(256) k_f2_reduce(F2Args a, int p, int nblocks, double *part2)
+// After the pass. blockIdx.z = 0: the listed particles. z = 1 .. 3, component
+// z - 1: part2[split][component][node] = sum over the split's workgroups, in
+// order, of the rows they hold of the node's row. The two are independent (the
+// listed particles' currents go to a.stray, which the next kernel adds), and
+// the listed ones take the longer for all that they are few: one particle's
+// gathers and pushes wait on memory one after another. In two launches, then in
+// this one (us a step): 48 x 36, 150,000 particles 66.5, 64.5; 64 x 64,
+// 2,000,000 particles 266, 256; 16,777,216 1639, 1622.
+template <int P, int MODE>
+__global__ void __launch_bounds__(256) k_f2_rest(F2Args a, int nblocks, double *part2)
 {
-    const int nn = a.nx * a.ny, c = blockIdx.z, splits = gridDim.y, sp = blockIdx.y;
+    const int nn = a.nx * a.ny, splits = gridDim.y, sp = blockIdx.y;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k == 0 && c == 0 && sp == 0) {
-        a.flags[1] += a.flags[2];
-        a.flags[2] = 0;
+    if (blockIdx.z == 0) {
+        const int n = a.flags[2], threads = gridDim.x * splits * blockDim.x;
+        int errs = 0;
+        for (int t = sp * gridDim.x * blockDim.x + k; t < n; t += threads) {
+            const int it = a.list[t];
+            errs |= f2_general<P, MODE>(a, it & 0x1fffffff, it >> 29);
+        }
+        if (errs) atomicOr(a.flags, errs);
+        return;
     }
     if (k >= nn) return;
-    const int gy = k / a.nx, gx = k - gy * a.nx;
+    const int c = blockIdx.z - 1, gy = k / a.nx, gx = k - gy * a.nx;
     const int b0 = (int)((int64_t)sp * nblocks / splits), b1 = (int)((int64_t)(sp + 1) * nblocks / splits);
     double t = 0.0;
     const size_t bs = (size_t)3 * a.hr * a.nx;
     if (a.strips == 1) {
-        const double *q = a.part + ((size_t)c * a.hr + gy + p) * a.nx + gx;     // rows -p .. ny
-        const int alias = gy >= a.ny - p ? -a.ny : (gy == 0 ? a.ny : 0);
+        const double *q = a.part + ((size_t)c * a.hr + gy + P) * a.nx + gx;     // rows -P .. ny
+        const int alias = gy >= a.ny - P ? -a.ny : (gy == 0 ? a.ny : 0);
 #pragma unroll 8
         for (int b = b0; b < b1; ++b) {
             double v = q[b * bs];
@@ -626,14 +626,10 @@ __global__ void __launch_bounds__(256) k_f2_reduce(F2Args a, int p, int nblocks,
         }
     } else {
         for (int b = b0; b < b1; ++b) {
-            const int jlo = a.wg[3 * b] * a.h - a.m - p;
+            const int jlo = a.wg[3 * b] * a.h - a.m - P;
             for (int r = imod(gy - jlo, a.ny); r < a.hr; r += a.ny)
                 t += a.part[b * bs + ((size_t)c * a.hr + r) * a.nx + gx];
         }
-    }
-    if (sp == 0) {
-        t += a.stray[(size_t)c * nn + k];
-        a.stray[(size_t)c * nn + k] = 0.0;
     }
     part2[((size_t)sp * 3 + c) * nn + k] = t;
 }
