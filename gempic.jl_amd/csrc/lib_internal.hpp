@@ -304,10 +304,11 @@ namespace gl {
 // solver's own stream: compute_e_from_b!, compute_b_from_e!, E -= M1^{-1} j
 // (compute_e_from_j!) and compute_rho_from_e! (maxwell_2d_fem.jl:370-499)
 hipStream_t m2d_stream(gempic_maxwell2d *m);
-// (with es, where m2d_fused: also es = E before + E after)
-void m2d_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *const *e,
-                  double *const *es = nullptr);
+void m2d_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *const *e);
 void m2d_b_from_e(gempic_maxwell2d *m, double dt, double *const *e, double *const *b);
+// the field work between two Strang steps (m2d_fused grids): HE's update of B,
+// HB twice in one with es = E before + E after, HE's update of B
+void m2d_between_steps(gempic_maxwell2d *m, double dt, double *const *b, double *const *e, double *const *es);
 void m2d_e_from_j(gempic_maxwell2d *m, const double *j, int component, double *e);
 // j = (sum of the partial grids part2[0 .. splits - 1], in order) * scale,
 // then e -= the inverse 1-form mass of j's component; false (nothing

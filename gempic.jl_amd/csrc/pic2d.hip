@@ -760,17 +760,32 @@ __global__ void k_sub(Field2 f, double *e, const double *w)
     FOR_NODES(f) e[k] = e[k] - w[k];
 }
 
-// compute_b_from_e! 2D (maxwell_2d_fem.jl:423-444)
+// compute_b_from_e! 2D (maxwell_2d_fem.jl:423-444): component c at node (i, j)
+// from the value b before
+__device__ __forceinline__ double b_from_e(const Field2 &f, int c, double dt, const double *e1, const double *e2,
+                                           const double *e3, int i, int j, double b)
+{
+    const int64_t k = i + (int64_t)j * f.nx;
+    const int64_t k1 = (i == 0 ? f.nx - 1 : i - 1) + (int64_t)j * f.nx;
+    const int64_t k2 = i + (int64_t)(j == 0 ? f.ny - 1 : j - 1) * f.nx;
+    if (c == 0) return b + -dt * (e3[k] - e3[k2]) / f.dy;
+    if (c == 1) return b + dt * (e3[k] - e3[k1]) / f.dx;
+    return b + -dt * ((e2[k] - e2[k1]) / f.dx - (e1[k] - e1[k2]) / f.dy);
+}
+
+// b = bs + the update (bs: b itself, or where k_fb_rows left it)
+struct FieldB {
+    const double *bs[3];
+    double *b[3];
+};
+
 __global__ void k_b_from_e(Field2 f, double dt, const double *e1, const double *e2,
-                           const double *e3, double *b1, double *b2, double *b3)
+                           const double *e3, FieldB a)
 {
     FOR_NODES(f) {
         const int i = (int)(k % f.nx), j = (int)(k / f.nx);
-        const int64_t k1 = (i == 0 ? f.nx - 1 : i - 1) + (int64_t)j * f.nx;
-        const int64_t k2 = i + (int64_t)(j == 0 ? f.ny - 1 : j - 1) * f.nx;
-        b1[k] += -dt * (e3[k] - e3[k2]) / f.dy;
-        b2[k] += dt * (e3[k] - e3[k1]) / f.dx;
-        b3[k] += -dt * ((e2[k] - e2[k1]) / f.dx - (e1[k] - e1[k2]) / f.dy);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) a.b[c][k] = b_from_e(f, c, dt, e1, e2, e3, i, j, a.bs[c][k]);
     }
 }
 
@@ -794,6 +809,9 @@ __global__ void k_div(Field2 f, const double *w1, const double *w2, double *rho)
 // kernels of host_inv_mass_kernel, applied as circular convolutions.
 
 constexpr int kFieldRows = 4, kFieldCols = 4, kFieldThreads = 256;
+// threads of k_fb_rows, which works on 4 rows and 7 around them: 256, 512 and
+// 1024 took 64.6, 63.2 and 62.1 us a step (2D3V, 150,000 particles, 48 x 36)
+constexpr int kFieldRowThreads = 1024;
 
 struct FieldTabs {
     const double *l0x, *l1x, *l0y, *l1y;   // mass lines of degree p and p - 1 (times dx, dy)
@@ -809,6 +827,7 @@ __device__ void conv_rows(const double *in, const double *k, int rows, int nx, d
         const double *line = in + rr * nx;
         double acc = 0.0;
         int u = i;
+#pragma unroll 8            // the LDS reads of eight terms in flight
         for (int m = 0; m < nx; ++m) {
             acc = __builtin_fma(k[m], line[u], acc);
             u = u == 0 ? nx - 1 : u - 1;
@@ -910,6 +929,7 @@ __global__ void __launch_bounds__(kFieldThreads) k_f_cols(Field2 f, FieldCols a,
         const double *line = col + cc * ny;
         double acc = 0.0;
         int u = j;
+#pragma unroll 8
         for (int m = 0; m < ny; ++m) {
             acc = __builtin_fma(kk[m], line[u], acc);
             u = u == 0 ? ny - 1 : u - 1;
@@ -923,9 +943,10 @@ __global__ void __launch_bounds__(kFieldThreads) k_f_cols(Field2 f, FieldCols a,
 
 // rows of a mass product M(x: lx, dgx; y: ly, dgy) b for the output rows
 // r0 .. r0 + nout - 1 (mod ny), with k_mass's arithmetic: the rows of b
-// from r0 - p (H = nout + 2p of them) staged in sb, their products along x
-// in mx, then along y into u
-__device__ void mass_rows(const double *b, const double *lx, int dgx, const double *ly, int dgy, int p,
+// from r0 - p (H = nout + 2p of them; b(i, j, row from r0)) staged in sb,
+// their products along x in mx, then along y into u
+template <class B>
+__device__ void mass_rows(B b, const double *lx, int dgx, const double *ly, int dgy, int p,
                           int r0, int nout, int nx, int ny, double *sb, double *mx, double *u)
 {
     const int H = nout + 2 * p;
@@ -933,7 +954,7 @@ __device__ void mass_rows(const double *b, const double *lx, int dgx, const doub
         const int hr = t / nx, i = t - hr * nx;
         int j = r0 - p + hr;
         j = j < 0 ? j + ny : (j >= ny ? j - ny : j);
-        sb[t] = b[(size_t)j * nx + i];
+        sb[t] = b(i, j, hr - p);
     }
     __syncthreads();
     for (int t = threadIdx.x; t < H * nx; t += blockDim.x) {
@@ -962,13 +983,20 @@ __device__ void mass_rows(const double *b, const double *lx, int dgx, const doub
 // compute_e_from_b! (maxwell_2d_fem.jl:370-411), first kernel: component
 // blockIdx.y of curl(M2 b) on the rows r0 .. r0 + rows - 1 (the mass
 // products and the curl of k_mass and k_curl_b), then its inverse mass
-// along x into tmp[c]
+// along x into tmp[c]. UPDATE: first b = b + compute_b_from_e!(dt_b, e) at the
+// rows as they are staged, each workgroup's own also written to bn (other
+// workgroups still read b); as a launch before this one the update took 3.1 us
+// and a gap of a step's 62 at 150,000 particles.
 struct FieldRowsB {
     const double *b[3];
     double *tmp[3];
+    const double *e[3];
+    double *bn[3];
+    double dt_b;
 };
 
-__global__ void __launch_bounds__(kFieldThreads) k_fb_rows(Field2 f, FieldTabs t, FieldRowsB a)
+template <bool UPDATE>
+__global__ void __launch_bounds__(kFieldRowThreads) k_fb_rows(Field2 f, FieldTabs t, FieldRowsB a)
 {
     extern __shared__ __align__(16) double lds[];
     const int nx = f.nx, ny = f.ny, p = t.degree, c = blockIdx.y;
@@ -978,12 +1006,23 @@ __global__ void __launch_bounds__(kFieldThreads) k_fb_rows(Field2 f, FieldTabs t
     double *cu = u2 + (kFieldRows + 1) * nx, *kk = cu + kFieldRows * nx;
     const double *kx = c == 0 ? t.k1x : t.k0x;
     for (int m = threadIdx.x; m < nx; m += blockDim.x) kk[m] = kx[m];
+    auto b = [&](int m) {
+        return [&, m](int i, int j, int row) {
+            double v = a.b[m][(size_t)j * nx + i];
+            if constexpr (UPDATE) {
+                v = b_from_e(f, m, a.dt_b, a.e[0], a.e[1], a.e[2], i, j, v);
+                // (B's component 3 is staged for c = 0 and 1: written once)
+                if (c != 1 && row >= 0 && row < rows) a.bn[m][(size_t)j * nx + i] = v;
+            }
+            return v;
+        };
+    };
     // u at rows r0 .. r0 + rows (the curl's j + 1 included)
     if (c == 2) {
-        mass_rows(a.b[0], t.l0x, p, t.l1y, p - 1, p, r0, rows + 1, nx, ny, sb, mx, u1);
-        mass_rows(a.b[1], t.l1x, p - 1, t.l0y, p, p, r0, rows + 1, nx, ny, sb, mx, u2);
+        mass_rows(b(0), t.l0x, p, t.l1y, p - 1, p, r0, rows + 1, nx, ny, sb, mx, u1);
+        mass_rows(b(1), t.l1x, p - 1, t.l0y, p, p, r0, rows + 1, nx, ny, sb, mx, u2);
     } else {
-        mass_rows(a.b[2], t.l1x, p - 1, t.l1y, p - 1, p, r0, rows + 1, nx, ny, sb, mx, u1);
+        mass_rows(b(2), t.l1x, p - 1, t.l1y, p - 1, p, r0, rows + 1, nx, ny, sb, mx, u1);
     }
     for (int q = threadIdx.x; q < rows * nx; q += blockDim.x) {
         const int rr = q / nx, i = q - rr * nx;
@@ -1232,12 +1271,12 @@ bool fused_setup(gempic_maxwell2d *m)
 {
     if ((int64_t)m->nx * m->ny > kFusedNodes) return false;
     const size_t shb = fb_rows_lds(m), shc = f_cols_lds(m);
-    if (shb > 65536 &&
-        hipFuncSetAttribute((const void *)k_fb_rows, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shb) !=
-            hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
+    if (shb > 65536)
+        for (const void *k : {(const void *)k_fb_rows<false>, (const void *)k_fb_rows<true>})
+            if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shb) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
     if (shc > 65536 &&
         hipFuncSetAttribute((const void *)k_f_cols, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shc) !=
             hipSuccess) {
@@ -1265,20 +1304,43 @@ hipStream_t gl::m2d_stream(gempic_maxwell2d *m) { return m->stream; }
 
 bool gl::m2d_fused(const gempic_maxwell2d *m) { return m->fused; }
 
-void gl::m2d_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *const *e, double *const *es)
+namespace {
+
+// compute_e_from_b! by the row and column kernels; with bn, b + the update by
+// compute_b_from_e!(dt_b, e) stands for b and is left in bn; with es, es = e
+// before + e after
+void fused_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *const *e, double *const *es,
+                    double dt_b, double *const *bn)
 {
     const Field2 f = m->f();
-    if (m->fused) {
-        const FieldTabs t = field_tabs(m);
-        FieldRowsB ra{{b[0], b[1], b[2]}, {m->buf(9), m->buf(10), m->buf(11)}};
-        hipLaunchKernelGGL(k_fb_rows, dim3((m->ny + kFieldRows - 1) / kFieldRows, 3), dim3(kFieldThreads),
-                           fb_rows_lds(m), m->stream, f, t, ra);
-        FieldCols ca{{m->buf(9), m->buf(10), m->buf(11)}, {t.k0y, t.k1y, t.k0y}, {e[0], e[1], e[2]},
-                     {es ? es[0] : nullptr, es ? es[1] : nullptr, es ? es[2] : nullptr}};
-        hipLaunchKernelGGL(k_f_cols, dim3((m->nx + kFieldCols - 1) / kFieldCols, 3), dim3(kFieldThreads),
-                           f_cols_lds(m), m->stream, f, ca, dt);
-        return;
+    const FieldTabs t = field_tabs(m);
+    FieldRowsB ra{{b[0], b[1], b[2]}, {m->buf(9), m->buf(10), m->buf(11)}, {e[0], e[1], e[2]}, {}, dt_b};
+    const dim3 grid((m->ny + kFieldRows - 1) / kFieldRows, 3), block(kFieldRowThreads);
+    if (bn) {
+        for (int c = 0; c < 3; ++c) ra.bn[c] = bn[c];
+        hipLaunchKernelGGL(k_fb_rows<true>, grid, block, fb_rows_lds(m), m->stream, f, t, ra);
+    } else {
+        hipLaunchKernelGGL(k_fb_rows<false>, grid, block, fb_rows_lds(m), m->stream, f, t, ra);
     }
+    FieldCols ca{{m->buf(9), m->buf(10), m->buf(11)}, {t.k0y, t.k1y, t.k0y}, {e[0], e[1], e[2]},
+                 {es ? es[0] : nullptr, es ? es[1] : nullptr, es ? es[2] : nullptr}};
+    hipLaunchKernelGGL(k_f_cols, dim3((m->nx + kFieldCols - 1) / kFieldCols, 3), dim3(kFieldThreads),
+                       f_cols_lds(m), m->stream, f, ca, dt);
+}
+
+void launch_b_from_e(gempic_maxwell2d *m, double dt, double *const *e, double *const *bs, double *const *b)
+{
+    const unsigned gb = grid_blocks((int64_t)m->nx * m->ny);
+    hipLaunchKernelGGL(k_b_from_e, dim3(gb), dim3(256), 0, m->stream, m->f(), dt, e[0], e[1], e[2],
+                       FieldB{{bs[0], bs[1], bs[2]}, {b[0], b[1], b[2]}});
+}
+
+}  // namespace
+
+void gl::m2d_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *const *e)
+{
+    if (m->fused) return fused_e_from_b(m, dt, b, e, nullptr, 0.0, nullptr);
+    const Field2 f = m->f();
     const unsigned gb = grid_blocks((int64_t)m->nx * m->ny);
     mass2(m, false, true, b[0], m->buf(6));
     mass2(m, true, false, b[1], m->buf(7));
@@ -1293,9 +1355,14 @@ void gl::m2d_e_from_b(gempic_maxwell2d *m, double dt, double *const *b, double *
 
 void gl::m2d_b_from_e(gempic_maxwell2d *m, double dt, double *const *e, double *const *b)
 {
-    const unsigned gb = grid_blocks((int64_t)m->nx * m->ny);
-    hipLaunchKernelGGL(k_b_from_e, dim3(gb), dim3(256), 0, m->stream, m->f(), dt, e[0], e[1], e[2],
-                       b[0], b[1], b[2]);
+    launch_b_from_e(m, dt, e, b, b);
+}
+
+void gl::m2d_between_steps(gempic_maxwell2d *m, double dt, double *const *b, double *const *e, double *const *es)
+{
+    double *bn[3] = {m->buf(6), m->buf(7), m->buf(8)};
+    fused_e_from_b(m, 2.0 * dt, b, e, es, dt, bn);
+    launch_b_from_e(m, dt, e, bn, b);
 }
 
 void gl::m2d_e_from_j(gempic_maxwell2d *m, const double *j, int component, double *e)
@@ -1526,8 +1593,8 @@ int gempic_maxwell2d_compute_b_from_e(gempic_maxwell2d *m, double dt, const doub
     const unsigned gb = grid_blocks((int64_t)m->nx * m->ny);
     H2D(m->buf(0), e1); H2D(m->buf(1), e2); H2D(m->buf(2), e3);
     H2D(m->buf(3), b1); H2D(m->buf(4), b2); H2D(m->buf(5), b3);
-    hipLaunchKernelGGL(k_b_from_e, dim3(gb), dim3(256), 0, m->stream, m->f(), dt, m->buf(0),
-                       m->buf(1), m->buf(2), m->buf(3), m->buf(4), m->buf(5));
+    hipLaunchKernelGGL(k_b_from_e, dim3(gb), dim3(256), 0, m->stream, m->f(), dt, m->buf(0), m->buf(1), m->buf(2),
+                       FieldB{{m->buf(3), m->buf(4), m->buf(5)}, {m->buf(3), m->buf(4), m->buf(5)}});
     D2H(b1, m->buf(3)); D2H(b2, m->buf(4)); D2H(b3, m->buf(5));
     return finish2(m);
 }

@@ -1325,9 +1325,7 @@ int gempic_splitting2d_strang_splitting(gempic_splitting2d *h, double dt, int64_
             if (s + 1 < n_steps) {
                 if (!rc) rc = f2_pass(h, F2_ALL, dt, e);
                 if (rc) break;
-                m2d_b_from_e(h->m, hdt, h->d_e, h->d_b);
-                m2d_e_from_b(h->m, 2.0 * hdt, h->d_b, h->d_e, h->d_es);
-                m2d_b_from_e(h->m, hdt, h->d_e, h->d_b);
+                m2d_between_steps(h->m, hdt, h->d_b, h->d_e, h->d_es);
             } else {
                 if (!rc) rc = f2_pass(h, F2_FIRST, dt, e);
                 if (!rc) rc = f2_pass(h, F2_SECOND, dt, e);
