@@ -1275,18 +1275,13 @@ int run_boris(gempic_splitting *h, int ops, double dt_e, double dt_b, double dt_
     a.dtqm_hp2 = h->qm * 0.5 * dt_b;       // qm * 0.5 * dt
     a.dt_hp1 = dt_x;
     a.more = more;
+    a.rgroups = epi_groups(L.blocks);
     {
         ProfScope ps(h, prof_id);
-        hipError_t e = launch_boris(h->deg0, h->deg1, ops, a, L.blocks, boris_shmem_bytes((int)h->nx),
+        hipError_t e = launch_boris(h->deg0, h->deg1, ops, kind, a, L.blocks, boris_shmem_bytes((int)h->nx),
                                     h->stream);
         if (e != hipSuccess)
             return fail(GEMPIC_ERR_DEVICE, std::string("Boris pass launch: ") + hipGetErrorString(e));
-    }
-    if (ops & BO_PUSHX) {
-        ProfScope ps(h, 9);
-        hipError_t e = launch_boris_epi(kind, a, L.blocks, h->stream);
-        if (e != hipSuccess)
-            return fail(GEMPIC_ERR_DEVICE, std::string("Boris field launch: ") + hipGetErrorString(e));
     }
     return GEMPIC_OK;
 }

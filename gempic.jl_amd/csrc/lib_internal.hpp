@@ -147,9 +147,8 @@ enum BorisOps : int { BO_EPART = 1, BO_BPART = 2, BO_EPART2 = 4, BO_PUSHX = 8 };
 // staggering!, or a strang_splitting! step (a.more: the next step's B
 // update follows)
 enum BorisEpi : int { BE_J = 0, BE_STAGGER, BE_STEP };
-hipError_t launch_boris(int p0, int p1, int ops, const PassArgs &a, int blocks, size_t shmem,
+hipError_t launch_boris(int p0, int p1, int ops, int kind, const PassArgs &a, int blocks, size_t shmem,
                         hipStream_t s);
-hipError_t launch_boris_epi(int kind, const PassArgs &a, int pass_blocks, hipStream_t s);
 size_t boris_shmem_bytes(int nx);
 int boris_blocks_per_cu(int p0, int p1, size_t shmem);
 

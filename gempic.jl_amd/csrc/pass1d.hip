@@ -1063,6 +1063,21 @@ int epi_groups(int nblocks)
     return g < 1 ? 1 : (g > kEpiGroupsMax ? kEpiGroupsMax : g);
 }
 
+// A pass's workgroup g of nblocks ends, its partial row stored by put_row<true>:
+// the last of a group sums the group's rows (with one group, nothing is summed
+// yet). Whether this is the last of all, which then reads the rows that are
+// left, by get_row<true>. Called by all threads; `flag` is shared.
+__device__ __forceinline__ bool last_of_pass(const PassArgs &a, int nblocks, int g, int ng, unsigned mask,
+                                             double *scratch, int spread_rows, int *flag)
+{
+    const int grp = ((g + 1) * ng - 1) / nblocks;          // the group with row g
+    const int b0 = (int)(((long)nblocks * grp) / ng), b1 = (int)(((long)nblocks * (grp + 1)) / ng);
+    if (!arrive_last(&a.cnt[1 + grp], (unsigned)(b1 - b0), flag)) return false;
+    if (ng == 1) return true;
+    sum_rows_range<true, true>(a.part, b0, b1, a.nx, mask, a.gpart + (size_t)grp * NDEP * a.nx, scratch, spread_rows);
+    return arrive_last(&a.cnt[0], (unsigned)ng, flag);
+}
+
 // PHASE 1: only workgroup g's sum of its group of rows into its group row;
 // PHASE 2: only the part after those sums (a later launch); PHASE 3: both, by
 // the pass's own workgroups (g: this one, of nblocks) as they end.
@@ -1111,20 +1126,10 @@ __device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g
         return;
     }
 
-    const double *last_rows = a.gpart;
-    int last_n = ng;
-    if constexpr (PHASE == 3) {
-        const int grp = ((g + 1) * ng - 1) / nblocks;          // the group with row g
-        const int b0 = (int)(((long)nblocks * grp) / ng), b1 = (int)(((long)nblocks * (grp + 1)) / ng);
-        if (!arrive_last(&a.cnt[1 + grp], (unsigned)(b1 - b0), &s_last)) return;
-        if (ng > 1) {
-            sum_rows_range<true, true>(a.part, b0, b1, nx, REDMASK, a.gpart + (size_t)grp * len, scratch, SPREAD);
-            if (!arrive_last(&a.cnt[0], (unsigned)ng, &s_last)) return;
-        } else {
-            last_rows = a.part;
-            last_n = nblocks;
-        }
-    }
+    if constexpr (PHASE == 3)
+        if (!last_of_pass(a, nblocks, g, ng, REDMASK, scratch, SPREAD, &s_last)) return;
+    const double *last_rows = PHASE == 3 && ng == 1 ? a.part : a.gpart;
+    const int last_n = PHASE == 3 && ng == 1 ? nblocks : ng;
     // The fields and the tables used are loaded into registers, so that they
     // arrive with the rows: nx <= kNxMax <= kBlock.
     static_assert(kNxMax <= kBlock, "one node per thread");
@@ -1598,7 +1603,117 @@ hipError_t launch_pass(int p0, int p1, int mode, const PassArgs &a, int blocks, 
 // position moves and the currents are deposited at the midpoint. OPS selects
 // the pushers for the stand-alone verbs.
 // ---------------------------------------------------------------------------
-template <int P0, int P1, int OPS>
+// The field part after a Boris x push, in the workgroup of the pass that ends
+// last (as epi1d_body): the deposit sum over the workgroups' rows, then
+//  BE_J:       j_dofs = the deposits (push_x_accumulate_j!);
+//  BE_STAGGER: staggering! (:103-121) with h = a.dt_hp1: E_mid = E,
+//              j = h j, E1_mid -= M1^-1 j1/dx, E2_mid += h W(B),
+//              E2_mid -= M0^-1 j2/dx;
+//  BE_STEP:    strang_splitting! (:158-175) with dt = a.dt_hp1: E = E_mid,
+//              j = dt j, the same E_mid updates with dt, and with a.more the
+//              next step's B_mid = (B + b_from_e(B, dt, E2_mid)) / 2 (:138-144).
+// As a launch of its own, and here (us a step): 60,000 particles 17.1, 17.1;
+// 300,001 23.2, 21.5; 1,048,576 29.6, 29.3.
+template <int KIND>
+__device__ __forceinline__ void boris_epi(const PassArgs &a, int nblocks, int g, int ng, double *smem)
+{
+    __shared__ int s_last;
+    constexpr unsigned REDMASK = (1u << D_J1) | (1u << D_J2A);
+    const int nx = a.nx;
+    const int tid = threadIdx.x;
+    const int nt = blockDim.x;
+    const int len = NDEP * nx;
+    const double dx = a.dx, h = a.dt_hp1;
+    double *sE1 = smem;                     // [nx] each: E1_mid (or E1), E2_mid (or E2), B, B_mid
+    double *sE2 = sE1 + nx;
+    double *sB = sE2 + nx;
+    double *sBM = sB + nx;
+    double *sRed = sBM + nx;                // [NDEP][nx]
+    double *work = sRed + NDEP * nx;
+    double *hc = work + nx;
+    double *T = hc + nx;                    // [NTAB][nx]
+    double *w3 = T + NTAB * nx;             // [6][nx]: outputs and workspaces of the solves
+    double *scratch = w3 + 6 * nx;          // [blockDim.x]
+    if (!last_of_pass(a, nblocks, g, ng, REDMASK, scratch, NDEP, &s_last)) return;
+    double *G = a.grid;
+    const int se1 = KIND == BE_STAGGER ? S_E1 : S_E1M, se2 = KIND == BE_STAGGER ? S_E2 : S_E2M;
+    // loaded into registers first, so that they arrive with the rows (as epi1d_body)
+    constexpr int TN = 5;                   // T_COS .. T_AMP
+    static_assert(T_AMP == T_COS + TN - 1, "contiguous tables");
+    double f_e1 = 0.0, f_e2 = 0.0, f_b = 0.0, f_t[TN];
+    if (tid < nx) {
+        f_e1 = G[se1 * nx + tid];
+        f_e2 = G[se2 * nx + tid];
+        f_b = G[S_B * nx + tid];
+#pragma unroll
+        for (int k = 0; k < TN; ++k) f_t[k] = a.tabs[(T_COS + k) * nx + tid];
+    }
+    for (int i = tid; i < len; i += nt) sRed[i] = 0.0;
+    __syncthreads();                        // sRed is zero
+    sum_rows_range<true>(ng == 1 ? a.part : a.gpart, 0, ng == 1 ? nblocks : ng, nx, REDMASK, sRed, scratch);
+    if (tid < nx) {
+        sE1[tid] = f_e1;
+        sE2[tid] = f_e2;
+        sB[tid] = f_b;
+#pragma unroll
+        for (int k = 0; k < TN; ++k) T[(T_COS + k) * nx + tid] = f_t[k];
+    }
+    __syncthreads();
+    double *r_j1 = sRed + D_J1 * nx, *r_j2 = sRed + D_J2A * nx;
+    if constexpr (KIND == BE_J) {
+        for (int i = tid; i < nx; i += nt) {
+            G[S_J1 * nx + i] = r_j1[i];
+            G[S_J2 * nx + i] = r_j2[i];
+        }
+        return;
+    } else {
+        for (int i = tid; i < nx; i += nt) {
+            if (KIND == BE_STEP) {               // e_dofs .= e_dofs_mid
+                G[S_E1 * nx + i] = sE1[i];
+                G[S_E2 * nx + i] = sE2[i];
+            }
+            r_j1[i] = h * r_j1[i];
+            r_j2[i] = h * r_j2[i];
+        }
+        __syncthreads();
+        // the three solves (M1^-1 j1, W(B), M0^-1 j2) are independent: run
+        // them side by side, then apply them in the reference's order
+        // (compute_e_from_j!(E1), compute_e_from_b!(E2), compute_e_from_j!(E2))
+        const SolveArgs s1{T + T_INVM1 * nx, r_j1, 1.0, w3, w3 + nx};
+        const SolveArgs sb{T + T_AMP * nx, sB, 1.0, w3 + 2 * nx, w3 + 3 * nx};
+        const SolveArgs s2{T + T_INVM0 * nx, r_j2, 1.0, w3 + 4 * nx, w3 + 5 * nx};
+        circ_solve3(s1, sb, s2, T + T_COS * nx, T + T_SIN * nx, nx);
+        const double coef = h / dx;
+        for (int i = tid; i < nx; i += nt) {
+            double w1 = s1.out[i] / dx;
+            sE1[i] -= w1;
+            sE2[i] += coef * sb.out[i];
+            double w2 = s2.out[i] / dx;
+            sE2[i] -= w2;
+        }
+        __syncthreads();
+        if (KIND == BE_STEP && a.more) {
+            for (int i = tid; i < nx; i += nt) sBM[i] = sB[i];
+            __syncthreads();
+            ep_b_from_e(sB, sE2, h, dx, nx);
+            for (int i = tid; i < nx; i += nt) sBM[i] = (sBM[i] + sB[i]) * 0.5;
+            __syncthreads();
+            for (int i = tid; i < nx; i += nt) {
+                G[S_B * nx + i] = sB[i];
+                G[S_BM * nx + i] = sBM[i];
+            }
+        }
+        for (int i = tid; i < nx; i += nt) {
+            G[S_J1 * nx + i] = r_j1[i];
+            G[S_J2 * nx + i] = r_j2[i];
+            G[S_E1M * nx + i] = sE1[i];
+            G[S_E2M * nx + i] = sE2[i];
+        }
+    }
+}
+
+// KIND: the field part that follows a PUSHX
+template <int P0, int P1, int OPS, int KIND>
 __global__ void __launch_bounds__(kBlock) k_boris1d(PassArgs a)
 {
     constexpr bool EPART = (OPS & BO_EPART) != 0;
@@ -1749,178 +1864,50 @@ __global__ void __launch_bounds__(kBlock) k_boris1d(PassArgs a)
             if (!((MASK >> r) & 1u)) continue;
             double t = 0.0;
             for (int wv = 0; wv < kWaves; ++wv) t += rows[wv * len + idx];
-            a.part[(size_t)blockIdx.x * len + idx] = t;
+            put_row<true>(&a.part[(size_t)blockIdx.x * len + idx], t);
         }
-    }
-}
-
-// The field part after a Boris x push: the deposit sum over the workgroups'
-// rows (group slices, then the last workgroup), then
-//  BE_J:       j_dofs = the deposits (push_x_accumulate_j!);
-//  BE_STAGGER: staggering! (:103-121) with h = a.dt_hp1: E_mid = E,
-//              j = h j, E1_mid -= M1^-1 j1/dx, E2_mid += h W(B),
-//              E2_mid -= M0^-1 j2/dx;
-//  BE_STEP:    strang_splitting! (:158-175) with dt = a.dt_hp1: E = E_mid,
-//              j = dt j, the same E_mid updates with dt, and with a.more the
-//              next step's B_mid = (B + b_from_e(B, dt, E2_mid)) / 2 (:138-144).
-template <int KIND>
-__global__ void __launch_bounds__(kBlock) k_boris_epi(PassArgs a, int nblocks)
-{
-    extern __shared__ double smem[];
-    __shared__ int s_last;
-    constexpr unsigned REDMASK = (1u << D_J1) | (1u << D_J2A);
-    const int nx = a.nx;
-    const int tid = threadIdx.x;
-    const int nt = blockDim.x;
-    const int len = NDEP * nx;
-    const double dx = a.dx, h = a.dt_hp1;
-    double *sE1 = smem;                     // [nx] each: E1_mid (or E1), E2_mid (or E2), B, B_mid
-    double *sE2 = sE1 + nx;
-    double *sB = sE2 + nx;
-    double *sBM = sB + nx;
-    double *sRed = sBM + nx;                // [NDEP][nx]
-    double *work = sRed + NDEP * nx;
-    double *hc = work + nx;
-    double *T = hc + nx;                    // [NTAB][nx]
-    double *w3 = T + NTAB * nx;             // [6][nx]: outputs and workspaces of the solves
-    double *scratch = w3 + 6 * nx;          // [blockDim.x]
-    double *G = a.grid;
-    const int se1 = KIND == BE_STAGGER ? S_E1 : S_E1M, se2 = KIND == BE_STAGGER ? S_E2 : S_E2M;
-    // loaded into registers first, so that they arrive with the rows (as epi1d_body)
-    constexpr int TN = 5;                   // T_COS .. T_AMP
-    static_assert(T_AMP == T_COS + TN - 1, "contiguous tables");
-    double f_e1 = 0.0, f_e2 = 0.0, f_b = 0.0, f_t[TN];
-    if (tid < nx) {
-        f_e1 = G[se1 * nx + tid];
-        f_e2 = G[se2 * nx + tid];
-        f_b = G[S_B * nx + tid];
-#pragma unroll
-        for (int k = 0; k < TN; ++k) f_t[k] = a.tabs[(T_COS + k) * nx + tid];
-    }
-    for (int i = tid; i < len; i += nt) sRed[i] = 0.0;
-    auto stage = [&] {
-        if (tid < nx) {
-            sE1[tid] = f_e1;
-            sE2[tid] = f_e2;
-            sB[tid] = f_b;
-#pragma unroll
-            for (int k = 0; k < TN; ++k) T[(T_COS + k) * nx + tid] = f_t[k];
-        }
-    };
-
-    const int ng = gridDim.x, g = blockIdx.x;
-    if (ng == 1) {
-        __syncthreads();                    // sRed is zero
-        sum_rows_range(a.part, 0, nblocks, nx, REDMASK, sRed, scratch);
-        stage();
-        __syncthreads();
-    } else {
-        sum_group_rows(a.part, nblocks, g, ng, nx, REDMASK, a.gpart + (size_t)g * len, scratch);
-        stage();
-        __threadfence();
-        __syncthreads();
-        if (tid == 0) s_last = atomicAdd(&a.cnt[0], 1u) == (unsigned)(ng - 1);
-        __syncthreads();
-        if (!s_last) return;
-        __threadfence();
-        if (tid == 0) a.cnt[0] = 0u;
-        sum_rows_range(a.gpart, 0, ng, nx, REDMASK, sRed, scratch);
-    }
-    double *r_j1 = sRed + D_J1 * nx, *r_j2 = sRed + D_J2A * nx;
-    if constexpr (KIND == BE_J) {
-        for (int i = tid; i < nx; i += nt) {
-            G[S_J1 * nx + i] = r_j1[i];
-            G[S_J2 * nx + i] = r_j2[i];
-        }
-        return;
-    } else {
-        for (int i = tid; i < nx; i += nt) {
-            if (KIND == BE_STEP) {               // e_dofs .= e_dofs_mid
-                G[S_E1 * nx + i] = sE1[i];
-                G[S_E2 * nx + i] = sE2[i];
-            }
-            r_j1[i] = h * r_j1[i];
-            r_j2[i] = h * r_j2[i];
-        }
-        __syncthreads();
-        // the three solves (M1^-1 j1, W(B), M0^-1 j2) are independent: run
-        // them side by side, then apply them in the reference's order
-        // (compute_e_from_j!(E1), compute_e_from_b!(E2), compute_e_from_j!(E2))
-        const SolveArgs s1{T + T_INVM1 * nx, r_j1, 1.0, w3, w3 + nx};
-        const SolveArgs sb{T + T_AMP * nx, sB, 1.0, w3 + 2 * nx, w3 + 3 * nx};
-        const SolveArgs s2{T + T_INVM0 * nx, r_j2, 1.0, w3 + 4 * nx, w3 + 5 * nx};
-        circ_solve3(s1, sb, s2, T + T_COS * nx, T + T_SIN * nx, nx);
-        const double coef = h / dx;
-        for (int i = tid; i < nx; i += nt) {
-            double w1 = s1.out[i] / dx;
-            sE1[i] -= w1;
-            sE2[i] += coef * sb.out[i];
-            double w2 = s2.out[i] / dx;
-            sE2[i] -= w2;
-        }
-        __syncthreads();
-        if (KIND == BE_STEP && a.more) {
-            for (int i = tid; i < nx; i += nt) sBM[i] = sB[i];
-            __syncthreads();
-            ep_b_from_e(sB, sE2, h, dx, nx);
-            for (int i = tid; i < nx; i += nt) sBM[i] = (sBM[i] + sB[i]) * 0.5;
-            __syncthreads();
-            for (int i = tid; i < nx; i += nt) {
-                G[S_B * nx + i] = sB[i];
-                G[S_BM * nx + i] = sBM[i];
-            }
-        }
-        for (int i = tid; i < nx; i += nt) {
-            G[S_J1 * nx + i] = r_j1[i];
-            G[S_J2 * nx + i] = r_j2[i];
-            G[S_E1M * nx + i] = sE1[i];
-            G[S_E2M * nx + i] = sE2[i];
-        }
+        boris_epi<KIND>(a, gridDim.x, blockIdx.x, a.rgroups, smem);
     }
 }
 
 size_t boris_shmem_bytes(int nx)
 {
-    return sizeof(double) * ((size_t)3 * (nx + 2 * kPad) + (size_t)kWaves * NDEP * nx +
-                             (size_t)kWaves * kSlotsPerLane * kWave);
-}
-
-static size_t boris_epi_shmem_bytes(int nx)
-{
-    return sizeof(double) * ((size_t)(4 + NDEP + 2 + NTAB + 6) * nx + kBlock);
+    const size_t pass = (size_t)3 * (nx + 2 * kPad) + (size_t)kWaves * NDEP * nx +
+                        (size_t)kWaves * kSlotsPerLane * kWave;
+    const size_t epi = (size_t)(4 + NDEP + 2 + NTAB + 6) * nx + kBlock;
+    return sizeof(double) * (pass > epi ? pass : epi);
 }
 
 template <int P0, int P1>
-static hipError_t launch_boris_pd(int ops, const PassArgs &a, int blocks, size_t shmem, hipStream_t s)
+static hipError_t launch_boris_pd(int ops, int kind, const PassArgs &a, int blocks, size_t shmem, hipStream_t s)
 {
-#define GK_BO(O)                                                                             \
-    case (O):                                                                                \
+#define GK_BO(O, K)                                                                          \
+    if (ops == (O) && kind == (K)) {                                                         \
         if (blocks < 0) {                                                                    \
             int nb = 0;                                                                      \
             hipError_t e_ = hipOccupancyMaxActiveBlocksPerMultiprocessor(                    \
-                &nb, k_boris1d<P0, P1, (O)>, kBlock, shmem);                                 \
+                &nb, k_boris1d<P0, P1, (O), (K)>, kBlock, shmem);                            \
             *(int *)a.diag = nb;                                                             \
             return e_;                                                                       \
         }                                                                                    \
-        hipLaunchKernelGGL((k_boris1d<P0, P1, (O)>), dim3(blocks), dim3(kBlock), shmem, s, a); \
-        return hipGetLastError();
-    switch (ops) {
-        GK_BO(BO_EPART | BO_BPART | BO_EPART2 | BO_PUSHX)
-        GK_BO(BO_PUSHX)
-        GK_BO(BO_EPART)
-        GK_BO(BO_BPART)
-    default:
-        return hipErrorInvalidValue;
+        hipLaunchKernelGGL((k_boris1d<P0, P1, (O), (K)>), dim3(blocks), dim3(kBlock), shmem, s, a); \
+        return hipGetLastError();                                                            \
     }
+    GK_BO(BO_EPART | BO_BPART | BO_EPART2 | BO_PUSHX, BE_STEP)
+    GK_BO(BO_PUSHX, BE_J)
+    GK_BO(BO_PUSHX, BE_STAGGER)
+    GK_BO(BO_EPART, BE_J)
+    GK_BO(BO_BPART, BE_J)
 #undef GK_BO
+    return hipErrorInvalidValue;
 }
 
-hipError_t launch_boris(int p0, int p1, int ops, const PassArgs &a, int blocks, size_t shmem,
+hipError_t launch_boris(int p0, int p1, int ops, int kind, const PassArgs &a, int blocks, size_t shmem,
                         hipStream_t s)
 {
-    if (a.nx > kNxMax) return hipErrorInvalidValue;
+    if (a.nx > kNxMax || blocks == 0) return hipErrorInvalidValue;
 #define GK_PAIR(A, B) \
-    if (p0 == (A) && p1 == (B)) return launch_boris_pd<A, B>(ops, a, blocks, shmem, s);
+    if (p0 == (A) && p1 == (B)) return launch_boris_pd<A, B>(ops, kind, a, blocks, shmem, s);
     GK_PAIR(1, 0)
     GK_PAIR(1, 1)
     GK_PAIR(2, 1)
@@ -1937,24 +1924,10 @@ int boris_blocks_per_cu(int p0, int p1, size_t shmem)
     int nb = 0;
     a.diag = (double *)&nb;
     a.nx = 1;
-    if (launch_boris(p0, p1, BO_EPART | BO_BPART | BO_EPART2 | BO_PUSHX, a, -1, shmem, nullptr) !=
+    if (launch_boris(p0, p1, BO_EPART | BO_BPART | BO_EPART2 | BO_PUSHX, BE_STEP, a, -1, shmem, nullptr) !=
             hipSuccess || nb < 1)
         return 1;
     return nb;
-}
-
-hipError_t launch_boris_epi(int kind, const PassArgs &a, int pass_blocks, hipStream_t s)
-{
-    if (a.nx > kNxMax || pass_blocks < 1) return hipErrorInvalidValue;
-    const dim3 grid(epi_groups(pass_blocks));
-    const size_t sh = boris_epi_shmem_bytes(a.nx);
-    switch (kind) {
-    case BE_J: hipLaunchKernelGGL(k_boris_epi<BE_J>, grid, dim3(kBlock), sh, s, a, pass_blocks); break;
-    case BE_STAGGER: hipLaunchKernelGGL(k_boris_epi<BE_STAGGER>, grid, dim3(kBlock), sh, s, a, pass_blocks); break;
-    case BE_STEP: hipLaunchKernelGGL(k_boris_epi<BE_STEP>, grid, dim3(kBlock), sh, s, a, pass_blocks); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
