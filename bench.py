@@ -7,9 +7,9 @@ solves in its last workgroup). Inputs are resident in GPU memory before the
 timed region starts.
 
 Prints one JSON line: particle-steps/s over the timed steps, the roofline of
-the fused pass (HIP-event kernel times on the library's stream, algorithmic
-56 bytes per particle-step: read x, v1, v2, w; write x, v1, v2), and a CPU
-baseline (the C oracle, one thread, on a bounded sample of the same workload).
+the fused pass with the field solves at its end (HIP-event kernel times on the
+library's stream, algorithmic 56 bytes per particle-step: read x, v1, v2, w;
+write x, v1, v2), and a CPU baseline (the C oracle, one thread, on a bounded sample of the same workload).
 """
 import argparse
 import json
@@ -67,22 +67,19 @@ def arith_run(G, _lib, w, arith, warmup, steps, blocks, interval, sort_s):
     if sort_s is not None and interval > 0:
         el += (steps / interval - (steps - 1) // interval) * sort_s
     ms, cnt = h.profile_read(0)
-    epi_ms, epi_cnt = h.profile_read(9)
     h.profile(False)
     pass_s = 1e-3 * ms / max(cnt, 1)
     ach = BYTES_FUSED * n / pass_s / 1e9
     del h
     return {"arithmetic": arith, "particles": n, "steps": steps,
             "value": n * steps / el, "ms_per_step": 1e3 * el / steps,
-            "pass_us": 1e6 * pass_s, "field_part_us": 1e3 * epi_ms / max(epi_cnt, 1),
+            "pass_us": 1e6 * pass_s,
             "roofline": {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": ach / HBM_PEAK_GBS, "bytes_per_particle_step": BYTES_FUSED}}
 
 
-BYTES_2D3V = 472          # per particle-step of the 2D3V splitting's passes: HE 64 x 2,
-                          # Hp3 64 x 2, Hp2 72 x 2, Hp1 72 (the state read: 40 B by HE,
-                          # 48 B with the weights by the others; the pushed components
-                          # written)
+BYTES_2D3V = 88           # per particle-step of the 2D3V splitting's fused pass: the state
+                          # and the weights read (48 B), the state written (40 B)
 
 
 def split2d_run(G, n, steps, cpu_n, cpu_steps):
@@ -292,7 +289,6 @@ def boris_run(G, _lib, w, steps, warmup):
     _lib.check(L.gempic_synchronize(h._h))
     elapsed = time.perf_counter() - t0
     pass_ms, pass_cnt = h.profile_read(0)
-    epi_ms, epi_cnt = h.profile_read(9)
     h.profile(False)
     pass_s = pass_ms / pass_cnt * 1e-3 if pass_cnt else float("nan")
     achieved = BYTES_FUSED * n / pass_s / 1e9
@@ -300,7 +296,6 @@ def boris_run(G, _lib, w, steps, warmup):
             "value": n * steps / elapsed, "unit": "particle-steps/s", "steps": steps,
             "ms_per_step": 1e3 * elapsed / steps,
             "pass_us": pass_s * 1e6,
-            "field_part_us": (epi_ms / epi_cnt * 1e3) if epi_cnt else None,
             "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                          "bytes_per_particle_step": BYTES_FUSED,
@@ -366,8 +361,7 @@ def adjoint_run(G, _lib, n, steps, every, cpu_n, cpu_steps):
     G.strang_splitting_adjoint_(h, dt, steps, checkpoint_every=every, fetch=False)
     t_adj = time.perf_counter() - t0
     kern = {}
-    for kid, name in ((0, "fused_pass"), (9, "deposit_sum_and_solves"), (10, "reverse_pass"),
-                      (11, "recompute_pass"), (12, "reverse_field_part")):
+    for kid, name in ((0, "fused_pass"), (10, "reverse_pass"), (11, "recompute_pass"), (12, "reverse_field_part")):
         ms, cnt = h.profile_read(kid)
         if cnt:
             kern[name] = {"avg_us": 1e3 * ms / cnt, "count": cnt}
@@ -671,7 +665,7 @@ def main():
     fused_ms, fused_cnt = h.profile_read(0)
     kernels = {}
     for kid, name in enumerate(["fused_pass", "trailing_pass", "he", "hp2", "hp1", "grid",
-                                "sort", "other", "fused_pass_a", "deposit_sum_and_solves"]):
+                                "sort", "other", "fused_pass_a"]):
         ms, cnt = h.profile_read(kid)
         if cnt:
             kernels[name] = {"avg_us": 1e3 * ms / cnt, "count": cnt}

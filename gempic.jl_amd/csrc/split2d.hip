@@ -7,9 +7,10 @@
 // degree per direction, and TwoDMaxwell's field operations
 // (maxwell_2d_fem.jl:370-499, run by pic2d.hip on device arrays). Fields:
 // E1 (p-1, p), E2 (p, p-1), E3 (p, p); B1 (p, p-1), B2 (p-1, p),
-// B3 (p-1, p-1). Particles: SoA x1, x2, v1, v2, v3, w, kept sorted by cell.
+// B3 (p-1, p-1). Particles: SoA x1, x2, v1, v2, v3, w.
 //
-// Each operator is one particle pass. A workgroup stages the fields it reads
+// A Strang step is one particle pass (step2d.hpp) on the grids that it takes;
+// else, and as a verb, each operator is one particle pass. A workgroup stages the fields it reads
 // in LDS, with a periodic halo of p nodes on the low side of each direction
 // (so a particle's stencil is constant offsets from its cell, no wrap), and
 // deposits its current into an LDS grid: each lane keeps the node sums of
