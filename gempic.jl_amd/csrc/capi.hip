@@ -103,9 +103,8 @@ struct Launch {
 //   1D1V (hot)    100,000: 46.1, 24.2, 24.3, 22.0   400,000: 40.8, 38.2, 33.2, 33.2
 //   24 instances of 65,536 to 524,288 particles in one ensemble, whose
 //   workgroups fill the chip together: 164, 175, 176, 181
-// An ensemble's instances keep their stand-alone partition (equal results),
-// so it pays for the small counts' gain; gempic_ensemble_autotune sets larger
-// chunks.
+// An ensemble's instances keep their stand-alone partition (equal results);
+// its pass takes several such blocks per workgroup (k_pass1d_batch).
 constexpr int kPerThread = 4;
 constexpr int kFewBlocks = 512;
 
@@ -1590,6 +1589,16 @@ int gempic_ensemble_destroy(gempic_ensemble *e)
 
 namespace {
 
+// Workgroups of an ensemble's pass at most, twice those that are on the chip
+// together: the second half evens out what the first ends at. us a step (24
+// instances, 65,536 to 524,288 particles) at 4, 8, 16 a CU and one workgroup
+// per block: 180, 172, 175, 183.
+constexpr int kEnsPerCu = 8;
+int ens_places(const gempic_ensemble *e)
+{
+    return e->hs[0]->cus * kEnsPerCu;
+}
+
 // the regular Strang step of an ensemble (another step follows, the previous
 // one's HE pending) as a graph: captured on the ensemble's stream, then
 // replayed; captured again when the launch geometry changed
@@ -1605,7 +1614,7 @@ int ens_step_graph(gempic_ensemble *e, const BatchArgs &b, int mode, size_t sh_p
     }
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-    const hipError_t e1 = launch_pass_batch(e->p0, e->p1, mode, b, e->bstart[ni], sh_pass, e->stream);
+    const hipError_t e1 = launch_pass_batch(e->p0, e->p1, mode, b, sh_pass, e->stream);
     const hipError_t e2 = launch_epi_batch(e->p0, e->p1, mode, b, e->estart[ni], sh_epi, e->stream);
     const hipError_t e3 = hipStreamEndCapture(e->stream, &g);
     if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
@@ -1670,12 +1679,14 @@ int gempic_ensemble_strang_splitting(gempic_ensemble *e, const double *dt, int64
         b.block_start = e->d_bstart;
         b.epi_start = e->d_estart;
         b.ninst = ni;
+        b.total = e->bstart[ni];
+        b.places = ens_places(e);
         if ((flags & GEMPIC_GRAPH) && s > 0 && s + 1 < n_steps) {
             rc = ens_step_graph(e, b, mode, sh_pass, sh_epi);
             if (rc) return rc;
             HIP_TRY(hipGraphLaunch(e->step_graph, e->stream));
         } else {
-            HIP_TRY(launch_pass_batch(e->p0, e->p1, mode, b, e->bstart[ni], sh_pass, e->stream));
+            HIP_TRY(launch_pass_batch(e->p0, e->p1, mode, b, sh_pass, e->stream));
             HIP_TRY(launch_epi_batch(e->p0, e->p1, mode, b, e->estart[ni], sh_epi, e->stream));
         }
         for (auto *h : e->hs) h->steps_since_sort++;
@@ -1686,7 +1697,9 @@ int gempic_ensemble_strang_splitting(gempic_ensemble *e, const double *dt, int64
     b.block_start = e->d_bstart;
     b.epi_start = e->d_estart;
     b.ninst = ni;
-    HIP_TRY(launch_pass_batch(e->p0, e->p1, M_HE_PREV | fast, b, e->bstart[ni],
+    b.total = e->bstart[ni];
+    b.places = ens_places(e);
+    HIP_TRY(launch_pass_batch(e->p0, e->p1, M_HE_PREV | fast, b,
                               pass_shmem_bytes(e->max_nx, M_HE_PREV), e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
     for (auto *h : e->hs) {
@@ -1912,13 +1925,15 @@ int gempic_ensemble_strang_splitting_adjoint(gempic_ensemble *e, const double *d
         b.block_start = e->d_bstart;
         b.epi_start = e->d_estart;
         b.ninst = ni;
+        b.total = e->bstart[ni];
+        b.places = ens_places(e);
         if (trailing) {
-            HIP_TRY(launch_pass_batch(e->p0, e->p1, M_HE_PREV, b, e->bstart[ni],
+            HIP_TRY(launch_pass_batch(e->p0, e->p1, M_HE_PREV, b,
                                       pass_shmem_bytes(e->max_nx, M_HE_PREV), e->stream));
             return GEMPIC_OK;
         }
         const int mode = (s > 1 ? M_HE_PREV : 0) | M_HE | M_HP2A | M_HP1 | M_HP2B;
-        HIP_TRY(launch_pass_batch(e->p0, e->p1, mode, b, e->bstart[ni], sh_pass, e->stream));
+        HIP_TRY(launch_pass_batch(e->p0, e->p1, mode, b, sh_pass, e->stream));
         HIP_TRY(launch_epi_batch(e->p0, e->p1, mode, b, e->estart[ni], sh_epi, e->stream));
         return GEMPIC_OK;
     };

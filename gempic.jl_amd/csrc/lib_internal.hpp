@@ -104,9 +104,10 @@ struct BatchArgs {
     const int *block_start;
     const int *epi_start;
     int ninst;
+    int total;       // blocks of all instances
+    int places;      // workgroups of the pass at most
 };
-hipError_t launch_pass_batch(int p0, int p1, int mode, const BatchArgs &b, int total_blocks,
-                             size_t shmem, hipStream_t s);
+hipError_t launch_pass_batch(int p0, int p1, int mode, const BatchArgs &b, size_t shmem, hipStream_t s);
 hipError_t launch_epi_batch(int p0, int p1, int mode, const BatchArgs &b, int total_groups,
                             size_t shmem, hipStream_t s);
 size_t epi_shmem_bytes(int nx);

@@ -507,10 +507,11 @@ template <int P0, int P1, int MODE, int PHASE>
 __device__ __forceinline__ void epi1d_body(const PassArgs &a, int nblocks, int g, int ng, double *smem);
 
 // ---------------------------------------------------------------------------
-// The particle pass; with TAIL, the workgroup that ends last runs the field
-// part (nblocks workgroups in all)
+// The particle pass of block bid; with TAIL, the workgroup that ends last runs
+// the field part (nblocks workgroups in all); with RUN, the blocks from bid up
+// to nblocks, one after another
 // ---------------------------------------------------------------------------
-template <int P0, int P1, int MODE, bool TAIL = false>
+template <int P0, int P1, int MODE, bool TAIL = false, bool RUN = false>
 __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *smem, int nblocks = 0)
 {
     constexpr bool HE_PREV = (MODE & M_HE_PREV) != 0;
@@ -551,14 +552,21 @@ __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *
 
     // this workgroup's chunk: particles base .. base + cnt_here - 1, addressed
     // through per-chunk base pointers and a 32-bit index
-    const PassChunk pc = pass_chunk(a, bid);
-    const int64_t base = pc.base;
-    const int cnt_here = pc.cnt;
-    const int iters = pc.iters;
-    double *__restrict__ px = a.x + base;
-    double *__restrict__ pv1 = a.v1 + base;
-    double *__restrict__ pv2 = a.v2 + base;
-    const double *__restrict__ pw = a.w + base;
+    int64_t base;
+    int cnt_here, iters;
+    double *__restrict__ px, *__restrict__ pv1, *__restrict__ pv2;
+    const double *__restrict__ pw;
+    auto set_chunk = [&] {
+        const PassChunk pc = pass_chunk(a, bid);
+        base = pc.base;
+        cnt_here = pc.cnt;
+        iters = pc.iters;
+        px = a.x + base;
+        pv1 = a.v1 + base;
+        pv2 = a.v2 + base;
+        pw = a.w + base;
+    };
+    set_chunk();
 
     // software pipeline: the loads of iteration it + kPrefetch are issued
     // before the work of iteration it; the first ones before the fields are
@@ -574,8 +582,11 @@ __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *
     };
     double nx_x = 0.0, nx_v1 = 0.0, nx_v2 = 0.0, nx_w = 0.0;     // iteration it + 1
     double n2_x = 0.0, n2_v1 = 0.0, n2_v2 = 0.0, n2_w = 0.0;     // it + 2 (kPrefetch 2)
-    if (iters > 0) load_particle(tid, nx_x, nx_v1, nx_v2, nx_w);
-    if (kPrefetch > 1 && iters > 1) load_particle(tid + kBlock, n2_x, n2_v1, n2_v2, n2_w);
+    auto load_first = [&] {
+        if (iters > 0) load_particle(tid, nx_x, nx_v1, nx_v2, nx_w);
+        if (kPrefetch > 1 && iters > 1) load_particle(tid + kBlock, n2_x, n2_v1, n2_v2, n2_w);
+    };
+    load_first();
 
     // E1 alone in 1d1v, none for the charge deposit
     if constexpr (!RHO_ONLY)
@@ -586,6 +597,11 @@ __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *
     __syncthreads();
     double *myrow = rows + wave * NDEP * nx;
 
+    const double xmin = a.xmin, dx = a.dx, qm = a.qm;
+    const double rdx = 1.0 / dx;     // div_by: (x - xmin) / dx, correctly rounded
+    bool e_inexact = false, e_far = false;   // error flags of this lane's particles
+
+    for (;;) {      // once, or (RUN) for each block bid .. nblocks - 1
     static_assert(W0 + W1 + W0 <= kSlotsPerLane, "cache-B slots");
     Cache2<W0> c_j2a;
     Cache2<W1> c_j1;
@@ -593,10 +609,6 @@ __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *
     if constexpr (HP2A) c_j2a.init(slots);
     if constexpr (HP1) c_j1.init(slots + W0 * kWave);
     if constexpr (NEED_NEW) c_new.init(slots + (W0 + W1) * kWave);
-
-    const double xmin = a.xmin, dx = a.dx, qm = a.qm;
-    const double rdx = 1.0 / dx;     // div_by: (x - xmin) / dx, correctly rounded
-    bool e_inexact = false, e_far = false;   // error flags of this lane's particles
 
     for (int it = 0; it < iters; ++it) {
         const int i = it * kBlock + tid;
@@ -830,8 +842,13 @@ __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *
                 a.cv2[base + i] = v2;
             }
     }
-    if (e_inexact || e_far) atomicOr(a.err, (e_inexact ? (int)E_INEXACT : 0) | (e_far ? (int)E_FAR : 0));
 
+    const int row = bid;
+    const bool more = RUN && ++bid < nblocks;
+    if (more) {
+        set_chunk();
+        load_first();
+    }
     if constexpr (DEPMASK != 0u) {
         if constexpr (HP2A) cache_drain<W0>(c_j2a, myrow + D_J2A * nx, nx);
         if constexpr (HP1) cache_drain<W1>(c_j1, myrow + D_J1 * nx, nx);
@@ -842,9 +859,18 @@ __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *
             const int r = (idx >= nx) + (idx >= 2 * nx) + (idx >= 3 * nx);
             if (!((DEPMASK >> r) & 1u)) continue;
             double s = 0.0;
-            for (int wv = 0; wv < kWaves; ++wv) s += rows[wv * len + idx];
-            put_row<TAIL>(&a.part[(size_t)bid * len + idx], s);
+            for (int wv = 0; wv < kWaves; ++wv) {
+                s += rows[wv * len + idx];
+                if (RUN) rows[wv * len + idx] = 0.0;
+            }
+            put_row<TAIL>(&a.part[(size_t)row * len + idx], s);
         }
+    }
+    if (RUN) __syncthreads();   // before the next block's deposits, or the next instance's fields
+    if (!more) break;
+    }
+    if (e_inexact || e_far) atomicOr(a.err, (e_inexact ? (int)E_INEXACT : 0) | (e_far ? (int)E_FAR : 0));
+    if constexpr (DEPMASK != 0u) {
         // the cross-workgroup sum and the field solves (the sub-steps' are the
         // same in either arithmetic)
         if constexpr (TAIL) {
@@ -885,15 +911,30 @@ __global__ void __launch_bounds__(kBlock, GEMPIC_PASS_MIN_WAVES) k_pass1d(PassAr
     pass1d_body<P0, P1, MODE, TAIL>(a, blockIdx.x, smem, gridDim.x);
 }
 
-// One launch runs the same pass for every instance of an ensemble; each
-// workgroup works for one instance with that instance's own launch geometry,
-// so every instance's result is the one its own launch would give.
+// One launch runs the same pass for every instance of an ensemble, each in the
+// blocks of its own launch geometry, so every instance's result is the one its
+// own launch would give. The blocks of small instances hold few particles, so a
+// workgroup takes several in turn, with the fields staged once and the next
+// block's first particles loaded before the drain. One block per workgroup, and
+// this (us a step): 24 instances of 65,536 to 524,288 particles 183, 172; 64 of
+// up to 1,048,576 746, 645, in the reference's arithmetic 825, 770.
 template <int P0, int P1, int MODE>
-__global__ void __launch_bounds__(kBlock) k_pass1d_batch(BatchArgs b)
+__global__ void __launch_bounds__(kBlock, GEMPIC_PASS_MIN_WAVES) k_pass1d_batch(BatchArgs b)
 {
     extern __shared__ double smem[];
-    const int inst = batch_instance(b.block_start, b.ninst, blockIdx.x);
-    pass1d_body<P0, P1, MODE>(b.args[inst], blockIdx.x - b.block_start[inst], smem);
+    // this workgroup's share of the batch's blocks, one instance's at a time
+    int first = (int)((int64_t)b.total * blockIdx.x / gridDim.x);
+    const int end = (int)((int64_t)b.total * (blockIdx.x + 1) / gridDim.x);
+    while (first < end) {
+        const int inst = batch_instance(b.block_start, b.ninst, first);
+        const int start = b.block_start[inst], next = b.block_start[inst + 1];
+        const int stop = end < next ? end : next;
+        // in the constant address space: read by scalar loads, also after the stores
+        using Args = const __attribute__((address_space(4))) PassArgs;
+        const PassArgs &a = *(const PassArgs *)((Args *)b.args + inst);
+        pass1d_body<P0, P1, MODE, false, true>(a, first - start, smem, stop - start);
+        first = stop;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1461,13 +1502,15 @@ template <int P0, int P1>
 static hipError_t launch_batch_pd(bool epi, int mode, const BatchArgs &b, int total, size_t shmem,
                                   hipStream_t s)
 {
+    const int places = total < b.places ? total : b.places;     // of the pass
+    if (!epi && places < 1) return hipErrorInvalidValue;
 #define GK_B(M)                                                                                  \
     case (M):                                                                                    \
         if (epi) {                                                                               \
             hipLaunchKernelGGL((k_epi1d_batch_sum<P0, P1, (M)>), dim3(total), dim3(kBlock), shmem, s, b); \
             hipLaunchKernelGGL((k_epi1d_batch_fin<P0, P1, (M)>), dim3(b.ninst), dim3(kBlock), shmem, s, b); \
         } else {                                                                                 \
-            hipLaunchKernelGGL((k_pass1d_batch<P0, P1, (M)>), dim3(total), dim3(kBlock), shmem, s, b); \
+            hipLaunchKernelGGL((k_pass1d_batch<P0, P1, (M)>), dim3(places), dim3(kBlock), shmem, s, b); \
         }                                                                                        \
         return hipGetLastError();
     switch (mode) {
@@ -1477,11 +1520,11 @@ static hipError_t launch_batch_pd(bool epi, int mode, const BatchArgs &b, int to
         GK_B(M_FAST | M_HE_PREV | M_HE | M_HP2A | M_HP1 | M_HP2B)
     case M_HE_PREV:
         if (epi) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((k_pass1d_batch<P0, P1, M_HE_PREV>), dim3(total), dim3(kBlock), shmem, s, b);
+        hipLaunchKernelGGL((k_pass1d_batch<P0, P1, M_HE_PREV>), dim3(places), dim3(kBlock), shmem, s, b);
         return hipGetLastError();
     case M_FAST | M_HE_PREV:
         if (epi) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((k_pass1d_batch<P0, P1, M_FAST | M_HE_PREV>), dim3(total), dim3(kBlock), shmem, s, b);
+        hipLaunchKernelGGL((k_pass1d_batch<P0, P1, M_FAST | M_HE_PREV>), dim3(places), dim3(kBlock), shmem, s, b);
         return hipGetLastError();
     default:
         return hipErrorInvalidValue;
@@ -1505,10 +1548,9 @@ static hipError_t launch_batch(bool epi, int p0, int p1, int mode, const BatchAr
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_pass_batch(int p0, int p1, int mode, const BatchArgs &b, int total_blocks,
-                             size_t shmem, hipStream_t s)
+hipError_t launch_pass_batch(int p0, int p1, int mode, const BatchArgs &b, size_t shmem, hipStream_t s)
 {
-    return launch_batch(false, p0, p1, mode, b, total_blocks, shmem, s);
+    return launch_batch(false, p0, p1, mode, b, b.total, shmem, s);
 }
 
 hipError_t launch_epi_batch(int p0, int p1, int mode, const BatchArgs &b, int total_groups,
