@@ -56,6 +56,32 @@ def test_gpu_ensemble_equals_standalone_runs():
         np.testing.assert_array_equal(h.b_dofs, ref[3])
 
 
+@pytest.mark.parametrize("arithmetic", ["reference", "fused"])
+def test_gpu_ensemble_with_several_blocks_per_workgroup(arithmetic):
+    """More blocks than the batched pass has workgroups (8 a CU: 2048), so that a
+    workgroup's run of blocks ends within instances and crosses from one into the
+    next (other nx, ragged last blocks, instances of one block): bit for bit each
+    instance's own run."""
+    specs = [(131072, 32, 1.1, 1), (130999, 16, 1.0, 2), (777, 16, 1.3, 3), (100, 64, 1.5, 4),
+             (131072, 64, 1.5, 5), (120001, 32, 1.25, 6), (131071, 16, 1.2, 7), (129000, 32, 1.0, 8)]
+    runs = []
+    for batched in (False, True):
+        hs = [_instance(n, nx, k, seed) for (n, nx, k, seed) in specs]
+        for h, _, _ in hs:
+            h.set_arithmetic(arithmetic)
+        if batched:
+            ens = G.Ensemble([h for h, _, _ in hs])
+            G.ensemble_strang_splitting_(ens, [_dt(nx) for (_, nx, _, _) in specs], 4)
+        else:
+            for (h, _, _), (_, nx, _, _) in zip(hs, specs):
+                G.strang_splitting_(h, _dt(nx), 4)
+        runs.append([(pg.array.copy(), h.e_dofs[0].copy(), h.e_dofs[1].copy(), h.b_dofs.copy())
+                     for h, pg, _ in hs])
+    for alone, batch in zip(*runs):
+        for a, b in zip(alone, batch):
+            np.testing.assert_array_equal(a, b)
+
+
 def test_gpu_ensemble_instance_matches_oracle_and_repeated_calls():
     h, pg, w = _instance(3000, 16, 1.25, 7)
     h2, pg2, _ = _instance(50000, 64, 1.0, 8)
