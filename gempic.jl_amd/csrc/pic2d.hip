@@ -880,10 +880,7 @@ __global__ void __launch_bounds__(kFieldThreads) k_fj_rows3(Field2 f, const doub
     const int r0 = blockIdx.x * kFieldRows, rows = min(kFieldRows, f.ny - r0);
     double *jr = lds, *kk = lds + kFieldRows * nx;
     const double *kx = a.kx[c];
-    if (blockIdx.x == 0 && c == 0 && threadIdx.x == 0) {     // count the listed particles, empty the list
-        a.flags[1] += a.flags[2];
-        a.flags[2] = 0;
-    }
+    if (blockIdx.x == 0 && c == 0 && threadIdx.x == 0) a.flags[1] = 0;      // empty the list
     for (int m = threadIdx.x; m < nx; m += blockDim.x) kk[m] = kx[m];
     for (int t = threadIdx.x; t < rows * nx; t += blockDim.x) {
         const int k = r0 * nx + t;

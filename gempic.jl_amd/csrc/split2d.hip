@@ -674,6 +674,18 @@ __global__ void k_s2_out(double *aos, int64_t ld, int64_t n, S2Perm pm)
 
 }  // namespace
 
+// The choice between the fused step and the operators' passes (f2_choose)
+struct F2Choice {
+    bool known = false;                     // `slow` was found for these particles and dt
+    bool slow = false;                      // too many would be listed: the operators' passes
+    bool pending = false;                   // a later prediction is under way
+    double dt = 0.0;
+    int64_t age = 0;                        // steps since the last prediction was queued
+    double scale = 1.0;                     // its sum -> listed particles a step
+    int *sums = nullptr;                    // [kPredictBlocks], pinned
+    hipEvent_t done = nullptr;
+};
+
 struct gempic_splitting2d {
     gempic_maxwell2d *m = nullptr;
     hipStream_t stream = nullptr;           // the solver's stream
@@ -700,10 +712,11 @@ struct gempic_splitting2d {
     // the fused step (step2d.hpp): its LDS layout, work arrays and the state
     // of the binning by strip
     bool f2 = false;                        // the grid takes it
-    bool f2_slow = false;                   // too many listed particles: the operators' passes instead
+    F2Choice choice;
     int f2_s = 0, f2_hr = 0, f2_strips = 1, f2_h = 0, f2_m = 0, f2_ntiles = 0;
     bool binned = false;
-    int64_t steps_since_bin = 0, f2_steps = 0;
+    int64_t steps_since_bin = 0;
+    int64_t fused_steps = 0, operator_steps = 0;    // run so far
     double *d_fpart = nullptr, *d_es[3] = {}, *d_stray = nullptr;
     int *d_bin = nullptr, *d_wg = nullptr, *d_list = nullptr;
 };
@@ -866,25 +879,13 @@ int s2_sort(gempic_splitting2d *h)
 // Steps between binnings by strip. Particles of the Landau configuration
 // drift 0.25 cells (rms) a step, 2.5 in ten, within the 5 rows to spare.
 constexpr int kBinEvery = 10;
-// The fused step's listed particles a step from which the operators' passes
-// are the faster way. A listed particle costs 6.5 ns; the fused step saves
-// 100 us a step at 150,000 particles (71 against 175), 300 at 4,000,000 (404
-// against 710), 700 at 16,777,216: the ways meet at 14 % (measured; 11.5 % by
-// this rule), 1.2 % (1.0 %) and 0.6 % (0.7 %) listed.
-constexpr double f2_listed_most(int64_t n) { return 16384.0 + (double)n / 160.0; }
-
 int s2_finish(gempic_splitting2d *h)
 {
     S2_TRY("2D3V splitting", hipStreamSynchronize(h->stream));
-    int flags[2] = {0, 0};                  // the error bits, the fused steps' listed particles
-    S2_TRY("2D3V splitting", hipMemcpy(flags, h->d_err, sizeof(flags), hipMemcpyDeviceToHost));
-    const int err = flags[0];
-    if (h->f2_steps > 0) {
-        if ((double)flags[1] > f2_listed_most(h->n) * (double)h->f2_steps) h->f2_slow = true;
-        h->f2_steps = 0;
-    }
-    if (flags[0] || flags[1]) S2_TRY("2D3V splitting", hipMemset(h->d_err, 0, sizeof(flags)));
+    int err = 0;
+    S2_TRY("2D3V splitting", hipMemcpy(&err, h->d_err, sizeof(int), hipMemcpyDeviceToHost));
     if (err) {
+        S2_TRY("2D3V splitting", hipMemset(h->d_err, 0, sizeof(int)));
         if (err & E_INEXACT)
             return abi_fail(GEMPIC_ERR_INEXACT, "InexactError: ceil(Int, x) of a non-finite or out-of-range position");
         return abi_fail(GEMPIC_ERR_INEXACT, "a particle crossed more than 65536 cells in one push");
@@ -980,6 +981,71 @@ F2Args f2_args(gempic_splitting2d *h, double dt)
     a.list = h->d_list;
     a.flags = h->d_err;
     return a;
+}
+
+// The fused step's listed particles a step from which the operators' passes
+// are the faster way. A listed particle costs 6.5 ns; the fused step saves
+// 100 us a step at 150,000 particles (71 against 175), 300 at 4,000,000 (404
+// against 710), 700 at 16,777,216: the ways meet at 14 % (measured; 11.5 % by
+// this rule), 1.2 % (1.0 %) and 0.6 % (0.7 %) listed.
+constexpr double f2_listed_most(int64_t n) { return 16384.0 + (double)n / 160.0; }
+// Steps between two predictions of it: with strips as often as the particles
+// are binned, since what they drift in that time counts.
+constexpr int kPredictEvery = 50;
+
+int f2_predict(gempic_splitting2d *h, double dt)
+{
+    F2Choice &c = h->choice;
+    const int64_t all = (h->n + kWave - 1) / kWave, stride = std::max<int64_t>(1, h->n / kPredictSample);
+    const int64_t groups = (all + stride - 1) / stride;
+    const int steps = h->f2_strips > 1 ? kBinEvery : 1;
+    hipLaunchKernelGGL(k_f2_predict, dim3(kPredictBlocks), dim3(1024), 0, h->stream, f2_args(h, dt), groups, stride,
+                       steps, c.sums);
+    S2_TRY("2D3V choice of path", hipGetLastError());
+    S2_TRY("2D3V choice of path", hipEventRecord(c.done, h->stream));
+    c.scale = (double)all / (double)groups / (double)steps;
+    c.dt = dt;
+    c.age = 0;
+    c.pending = true;
+    return GEMPIC_OK;
+}
+
+int f2_take(gempic_splitting2d *h)
+{
+    F2Choice &c = h->choice;
+    S2_TRY("2D3V choice of path", hipEventSynchronize(c.done));
+    int64_t sum = 0;
+    for (int k = 0; k < kPredictBlocks; ++k) sum += c.sums[k];
+    c.slow = (double)sum * c.scale > f2_listed_most(h->n);
+    c.known = true;
+    c.pending = false;
+    return GEMPIC_OK;
+}
+
+// Before a step by dt: whether it takes the operators' passes (slow). The first
+// step of new particles or of another dt waits for its own prediction. Later
+// ones are queued every few steps and looked at when the next is due, by when
+// the GPU is past them, so that it never waits: a call that ends with its
+// steps waits for that one rather than run further ahead of it (wait), one that
+// only queues them goes on as before while it is not there.
+int f2_choose(gempic_splitting2d *h, double dt, bool wait, bool &slow)
+{
+    F2Choice &c = h->choice;
+    slow = !h->f2 || h->n == 0;
+    if (slow || !c.sums) return GEMPIC_OK;
+    int rc = GEMPIC_OK;
+    if (!c.known || dt != c.dt) {
+        rc = f2_predict(h, dt);
+        if (!rc) rc = f2_take(h);
+    } else if (c.age >= (h->f2_strips > 1 ? kBinEvery : kPredictEvery)) {
+        if (c.pending) {
+            if (wait || hipEventQuery(c.done) == hipSuccess) rc = f2_take(h);
+            else (void)hipGetLastError();           // "not ready" is no error
+        }
+        if (!rc && !c.pending) rc = f2_predict(h, dt);
+    }
+    slow = c.slow;
+    return rc;
 }
 
 // particles by strip, and the ranges of the particle workgroups
@@ -1126,7 +1192,7 @@ int gempic_splitting2d_create(int64_t nx, int64_t ny, double xmin, double xmax, 
     }
     al((void **)&h->d_rho, sizeof(double) * nn);
     al((void **)&h->d_part, sizeof(double) * nn * (size_t)(h->blocks + kSplits2));
-    al((void **)&h->d_err, 3 * sizeof(int));
+    al((void **)&h->d_err, 2 * sizeof(int));
     h->f2 = f2_layout(h) && h->blocks > 2 * h->f2_strips;
     if (h->f2) {
         h->f2_ntiles = (int)((np + kBinTile - 1) / kBinTile);
@@ -1140,10 +1206,18 @@ int gempic_splitting2d_create(int64_t nx, int64_t ny, double xmin, double xmax, 
         for (int mode : {F2_ALL, F2_FIRST, F2_SECOND})
             if (e == hipSuccess && f2_shmem(h, mode) > 65536)
                 e = hipFuncSetAttribute(f2_kernel(degree, mode), hipFuncAttributeMaxDynamicSharedMemorySize, kF2Lds);
+        // (fewer particles than may be listed need no choice)
+        if ((double)np > f2_listed_most(n_particles)) {
+            if (e == hipSuccess)
+                e = hipHostMalloc((void **)&h->choice.sums, sizeof(int) * kPredictBlocks, hipHostMallocCoherent);
+            // (the sums go to coherent memory; a system fence per event cost 18 us)
+            if (e == hipSuccess)
+                e = hipEventCreateWithFlags(&h->choice.done, hipEventDisableTiming | hipEventDisableSystemFence);
+        }
     }
     al((void **)&h->d_count, sizeof(int) * nn);
     al((void **)&h->d_cursor, sizeof(int) * nn);
-    if (e == hipSuccess) e = hipMemset(h->d_err, 0, 3 * sizeof(int));
+    if (e == hipSuccess) e = hipMemset(h->d_err, 0, 2 * sizeof(int));
     for (int c = 0; c < 3 && e == hipSuccess; ++c) {
         e = hipMemset(h->d_e[c], 0, sizeof(double) * nn);
         if (e == hipSuccess) e = hipMemset(h->d_b[c], 0, sizeof(double) * nn);
@@ -1183,6 +1257,8 @@ int gempic_splitting2d_destroy(gempic_splitting2d *h)
                     h->d_bin, h->d_wg, h->d_list};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    if (h->choice.done) (void)hipEventDestroy(h->choice.done);
+    if (h->choice.sums) (void)hipHostFree(h->choice.sums);
     if (h->m) gempic_maxwell2d_destroy(h->m);
     transfer_release();
     delete h;
@@ -1207,7 +1283,7 @@ int gempic_splitting2d_set_particles(gempic_splitting2d *h, const double *aos, i
     S2_TRY("2D3V upload", hipGetLastError());
     h->steps_since_sort = 0;
     h->binned = false;
-    h->f2_slow = false;
+    h->choice.known = false;
     int rc = h->sort_interval > 0 ? s2_sort(h) : GEMPIC_OK;   // sorted on upload where sorting is on
     if (rc) return rc;
     return s2_finish(h);
@@ -1307,53 +1383,71 @@ int gempic_splitting2d_strang_splitting(gempic_splitting2d *h, double dt, int64_
     if (n_steps < 0) return abi_fail(GEMPIC_ERR_ARGUMENT, "ArgumentError: number_steps must be >= 0");
     const double hdt = 0.5 * dt;
     int rc = GEMPIC_OK;
-    const bool fused = h->f2 && !h->f2_slow && h->n > 0;
-    if (fused && n_steps > 0) {
-        // HB and HE's B update of the first step; then per step one particle
-        // pass and the field work up to the next step's. E after the
-        // currents is the last HE's field of this step, es = that plus E
-        // after both HB the field of the two HE of a step's end and the
-        // next's begin.
-        s2_hb(h, hdt);
-        m2d_b_from_e(h->m, hdt, h->d_e, h->d_b);
-        for (int64_t s = 0; s < n_steps && !rc; ++s) {
-            if (h->sort_interval > 0 && h->steps_since_sort >= h->sort_interval) {
-                rc = s2_sort(h);
-                h->binned = false;
+    // A fused step: HB and HE's B update of the first one; then per step one
+    // particle pass and the field work up to the next step's, which leaves the
+    // call `open`. E after the currents is the last HE's field of this step, es =
+    // that plus E after both HB the field of the two HE of a step's end and the
+    // next's begin. A step of the operators' passes after an open one has its
+    // two E kicks left to do.
+    bool open = false;
+    for (int64_t s = 0; s < n_steps && !rc; ++s) {
+        bool slow = true;
+        rc = f2_choose(h, dt, !(flags & GEMPIC_ASYNC), slow);
+        if (!rc && h->sort_interval > 0 && h->steps_since_sort >= h->sort_interval) {
+            rc = s2_sort(h);
+            h->binned = false;
+        }
+        if (!rc && slow) {
+            if (open) {
+                rc = s2_pass(h, S2_HE, hdt, h->d_es[0], h->d_es[1], h->d_es[2], nullptr, 1.0);
+            } else {
+                rc = s2_hb(h, hdt);
+                if (!rc) rc = s2_he(h, hdt);
             }
-            if (!rc && h->f2_strips > 1 && (!h->binned || h->steps_since_bin >= kBinEvery)) rc = f2_bin(h);
-            double *const *e = s == 0 ? h->d_e : h->d_es;
+            if (!rc) rc = s2_hp(h, 3, hdt);
+            if (!rc) rc = s2_hp(h, 2, hdt);
+            if (!rc) rc = s2_hp(h, 1, dt);
+            if (!rc) rc = s2_hp(h, 2, hdt);
+            if (!rc) rc = s2_hp(h, 3, hdt);
+            if (!rc) rc = s2_he(h, hdt);
+            if (!rc) rc = s2_hb(h, hdt);
+            open = false;
+            h->operator_steps++;
+        } else if (!rc) {
+            if (!open) {
+                s2_hb(h, hdt);
+                m2d_b_from_e(h->m, hdt, h->d_e, h->d_b);
+            }
+            double *const *e = open ? h->d_es : h->d_e;
+            if (h->f2_strips > 1 && (!h->binned || h->steps_since_bin >= kBinEvery)) rc = f2_bin(h);
             if (s + 1 < n_steps) {
                 if (!rc) rc = f2_pass(h, F2_ALL, dt, e);
                 if (rc) break;
                 m2d_between_steps(h->m, hdt, h->d_b, h->d_e, h->d_es);
+                open = true;
             } else {
                 if (!rc) rc = f2_pass(h, F2_FIRST, dt, e);
                 if (!rc) rc = f2_pass(h, F2_SECOND, dt, e);
                 if (!rc) rc = s2_he(h, hdt);
                 if (!rc) rc = s2_hb(h, hdt);
             }
-            h->steps_since_sort++;
-            h->steps_since_bin++;
-            h->f2_steps++;
+            h->fused_steps++;
         }
-    }
-    for (int64_t s = 0; s < n_steps && !rc && !fused; ++s) {
-        if (h->sort_interval > 0 && h->steps_since_sort >= h->sort_interval) rc = s2_sort(h);
-        if (!rc) rc = s2_hb(h, hdt);
-        if (!rc) rc = s2_he(h, hdt);
-        if (!rc) rc = s2_hp(h, 3, hdt);
-        if (!rc) rc = s2_hp(h, 2, hdt);
-        if (!rc) rc = s2_hp(h, 1, dt);
-        if (!rc) rc = s2_hp(h, 2, hdt);
-        if (!rc) rc = s2_hp(h, 3, hdt);
-        if (!rc) rc = s2_he(h, hdt);
-        if (!rc) rc = s2_hb(h, hdt);
+        h->choice.age++;
         h->steps_since_sort++;
+        h->steps_since_bin++;
     }
     if (rc) return rc;
     if (flags & GEMPIC_ASYNC) return GEMPIC_OK;
     return s2_finish(h);
+}
+
+int gempic_splitting2d_step_counts(gempic_splitting2d *h, int64_t *fused, int64_t *operators)
+{
+    CHECK_H2(h);
+    if (fused) *fused = h->fused_steps;
+    if (operators) *operators = h->operator_steps;
+    return GEMPIC_OK;
 }
 
 int gempic_splitting2d_synchronize(gempic_splitting2d *h)

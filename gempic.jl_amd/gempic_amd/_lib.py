@@ -127,6 +127,7 @@ SIGNATURES = {
     "gempic_splitting2d_operator_hp2": (_I, [_VP, _D]),
     "gempic_splitting2d_operator_hp3": (_I, [_VP, _D]),
     "gempic_splitting2d_strang_splitting": (_I, [_VP, _D, _I64, _I]),
+    "gempic_splitting2d_step_counts": (_I, [_VP, ctypes.POINTER(_I64), ctypes.POINTER(_I64)]),
     "gempic_splitting2d_synchronize": (_I, [_VP]),
     "gempic_splitting2d_set_sort_interval": (_I, [_VP, _I64]),
     "gempic_splitting2d_rho": (_I, [_VP, _P]),

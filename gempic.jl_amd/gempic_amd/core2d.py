@@ -623,6 +623,12 @@ class HamiltonianSplitting2D3V:
         self._run(_lib.load().gempic_splitting2d_strang_splitting, float(dt), int(number_steps),
                   16 if async_ else 0)
 
+    def step_counts(self) -> tuple:
+        """Strang steps so far that ran as one particle pass, and as the operators' passes."""
+        k = (ctypes.c_int64(), ctypes.c_int64())
+        check(_lib.load().gempic_splitting2d_step_counts(self._h, ctypes.byref(k[0]), ctypes.byref(k[1])))
+        return k[0].value, k[1].value
+
     def synchronize(self):
         check(_lib.load().gempic_splitting2d_synchronize(self._h))
 

@@ -535,8 +535,13 @@ int gempic_splitting2d_operator_he(gempic_splitting2d *h, double dt);
 int gempic_splitting2d_operator_hp1(gempic_splitting2d *h, double dt);
 int gempic_splitting2d_operator_hp2(gempic_splitting2d *h, double dt);
 int gempic_splitting2d_operator_hp3(gempic_splitting2d *h, double dt);
-/* flags: GEMPIC_ASYNC returns once the work is queued */
+/* flags: GEMPIC_ASYNC returns once the work is queued, but the first step of
+ * new particles or of another dt waits for the choice of its kernels. */
 int gempic_splitting2d_strang_splitting(gempic_splitting2d *h, double dt, int64_t n_steps, int flags);
+/* Strang steps so far that ran as one particle pass, and as the operators'
+ * passes: a step takes the latter while too many particles cross more than one
+ * cell in a push or drift far in a few steps. Either may be NULL. */
+int gempic_splitting2d_step_counts(gempic_splitting2d *h, int64_t *fused, int64_t *operators);
 int gempic_splitting2d_synchronize(gempic_splitting2d *h);
 /* sort the particles by cell every `interval` Strang steps (0, the default:
    never; the passes run faster on unordered particles) */

@@ -198,6 +198,72 @@ def test_gpu_2d3v_fused_steps_match_oracle(degree, nx, ny, n, vscale, steps):
             _close(h.j_dofs[c], osp.j(c + 1), 1e-11, f"j{c + 1}")
 
 
+def _same_state(h, pg, osp, o_parts, o_e, o_b, rel):
+    h.to_host()
+    for r in range(5):
+        _close(pg.array[r], o_parts[r], rel, f"row {r}")
+    for c in range(3):
+        _close(h.e_dofs[c], o_e[c], rel, f"E{c + 1}")
+        _close(h.b_dofs[c], o_b[c], rel, f"B{c + 1}")
+        _close(h.j_dofs[c], osp.j(c + 1), rel, f"j{c + 1}")
+
+
+@pytest.mark.parametrize("n, steps, fused", [(16000, 2, True), (40001, 13, False)])
+def test_gpu_2d3v_hot_particles_take_the_operators_passes(n, steps, fused):
+    """Particles that nearly all cross several cells in a push: from the first
+    call on the operators' passes, also after another upload and with another
+    dt. 16,000 particles, as many as a step may always list, take the one-pass
+    step's general form."""
+    print(f"2d3v hot: n={n}, {steps} steps", flush=True)
+    w = _hot(n=n, nx=64, ny=64, L1=16.0, L2=16.0, seed=9, vscale=20.0, fscale=0.05)
+    h, pg, osp, o_parts, o_e, o_b = _pair(w, 3, sync=False)
+    done = 0
+    for dt, k in ((0.05, steps), (0.05, 1), (0.04, 2)):
+        h.strang_splitting(dt, k)
+        osp.strang_splitting(dt, k)
+        done += k
+        _same_state(h, pg, osp, o_parts, o_e, o_b, 1e-10)
+        assert h.step_counts() == ((done, 0) if fused else (0, done))
+        h.to_device()
+
+
+@pytest.mark.parametrize("nx, ny, turn, calls", [(64, 64, 0.05, (80,)), (64, 64, 0.05, (1,) * 25 + (55,)),
+                                                (48, 36, 0.0125, (300,))])
+def test_gpu_2d3v_path_changes_within_a_call(nx, ny, turn, calls):
+    """A beam that a uniform B3 turns from x2 to x1 and on (`turn` a step): along
+    x1 it crosses 2.2 cells a step, along x2 a quarter. The step goes from one
+    pass to the operators' passes and back within a call (strips: looked at every
+    10 steps; whole grids in LDS: every 50), and the state and the currents stay
+    the oracle's. The charge is small, so rounding differences (3e-14 a step)
+    only add up."""
+    print(f"2d3v path changes: {nx} x {ny}, calls {calls}", flush=True)
+    n, dt = 20001, 0.05
+    w = _hot(n=n, nx=nx, ny=ny, L1=0.25 * nx, L2=2.0 * ny, seed=10, vscale=0.2, fscale=1e-3)
+    w["common_weight"] = 1e-8
+    w["particles"][3] += 11.0
+    w["b"][2] += turn / dt
+    h, pg, osp, o_parts, o_e, o_b = _pair(w, 3, sync=False)
+    for k in calls:
+        h.strang_splitting(dt, k)
+        osp.strang_splitting(dt, k)
+    fused, operators = h.step_counts()
+    print(f"   {fused} steps as one pass, {operators} as the operators' passes", flush=True)
+    assert fused + operators == sum(calls) and fused >= 20 and operators >= 20
+    _same_state(h, pg, osp, o_parts, o_e, o_b, 1e-11)
+
+
+def test_gpu_2d3v_queued_calls_match_oracle():
+    """Calls that only queue their steps, on particles that all cross several
+    cells, and a last one that waits."""
+    print("2d3v queued calls", flush=True)
+    w = _hot(n=20001, nx=64, ny=64, L1=16.0, L2=16.0, seed=11, vscale=20.0, fscale=0.05)
+    h, pg, osp, o_parts, o_e, o_b = _pair(w, 3, sync=False)
+    for k in range(25):
+        h.strang_splitting(0.05, 1, async_=k < 24)
+    osp.strang_splitting(0.05, 25)
+    _same_state(h, pg, osp, o_parts, o_e, o_b, 1e-10)
+
+
 def test_gpu_2d3v_errors_and_order():
     w = _hot(n=1000)
     h, pg, *_ = _pair(w, 3)
