@@ -276,22 +276,16 @@ struct Cache2 {
     double a[WN];
     double *bs;           // entry B: value w at bs[w * kWave] (this lane's LDS slots)
 
-    // slots: the wave's WN * kWave doubles of LDS for this cache
+    // slots: the wave's WN * kWave doubles of LDS for this cache; entry B's are
+    // cleared when it takes a cell, and not read before
     __device__ __forceinline__ void init(double *slots)
     {
         bs = slots + lane_id();
-        reset();
-    }
-    __device__ __forceinline__ void reset()
-    {
         ca = -1;
         cb = -1;
         mru_b = false;
 #pragma unroll
-        for (int w = 0; w < WN; ++w) {
-            a[w] = 0.0;
-            bs[w * kWave] = 0.0;
-        }
+        for (int w = 0; w < WN; ++w) a[w] = 0.0;
     }
 };
 
@@ -388,9 +382,10 @@ __device__ __forceinline__ void row_add(const double (&v)[WN], int cell, double 
     const int lane = lane_id();
     const int w = quad_value(lane >> 4);
     if ((lane & 15) == 0 && w < N) {
+        // node 1 - WN .. cell (a loop to 0 became a division of it)
         int k = cell - (WN - 1) + W0 + w;
-        while (k < 0) k += nx;
-        while (k >= nx) k -= nx;
+#pragma unroll
+        for (int t = 1; t < WN; ++t) k = k < 0 ? k + nx : k;
         __hip_atomic_fetch_add(&row[k], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     if constexpr (WN - W0 > 4) row_add<WN, W0 + 4>(v, cell, row, nx);
@@ -404,6 +399,11 @@ __device__ __forceinline__ void row_add(const double (&v)[WN], int cell, double 
 // splitting fell from 48.6 to 38.2 us at 16,384 particles and from 68.2 to
 // 63.7 us at 4,194,304, and one of the 1D1V splitting with 100,000 hot
 // particles, whose lanes flush many cells, from 77.4 to 55.6 us.
+// Small blocks pay for it with every few particles: with the nodes wrapped by
+// selects (a loop became a division) and entry B's LDS left alone where no lane
+// has one, 32 instances of 131,072 particles in one ensemble take 129 us a step
+// (143 before; 151 and 167 in the reference's arithmetic), 300,001 particles on 50
+// nodes 5 % less, 4,194,304 2 % less.
 template <int WN>
 __device__ __forceinline__ void seg_flush(bool want, int cell, const double (&v)[WN], double *row,
                                           int nx)
@@ -432,11 +432,13 @@ __device__ __forceinline__ void cache_add(Cache2<WN> &C, bool valid, int cell,
         bool use_b = miss && !use_a;
         bool ev_a = use_a && C.ca >= 0;
         bool ev_b = use_b && C.cb >= 0;
-        int ecell = ev_a ? C.ca : C.cb;
-        double ev[WN];
+        if (__ballot(ev_a || ev_b)) {
+            int ecell = ev_a ? C.ca : C.cb;
+            double ev[WN];
 #pragma unroll
-        for (int w = 0; w < WN; ++w) ev[w] = ev_a ? C.a[w] : C.bs[w * kWave];
-        seg_flush<WN>(ev_a || ev_b, ecell, ev, row, nx);
+            for (int w = 0; w < WN; ++w) ev[w] = ev_a ? C.a[w] : C.bs[w * kWave];
+            seg_flush<WN>(ev_a || ev_b, ecell, ev, row, nx);
+        }
         if (use_a) {
             C.ca = cell;
 #pragma unroll
@@ -468,11 +470,12 @@ template <int WN>
 __device__ __forceinline__ void cache_drain(Cache2<WN> &C, double *row, int nx)
 {
     seg_flush<WN>(C.ca >= 0, C.ca, C.a, row, nx);
-    double bv[WN];
+    if (__ballot(C.cb >= 0)) {
+        double bv[WN];
 #pragma unroll
-    for (int w = 0; w < WN; ++w) bv[w] = C.bs[w * kWave];
-    seg_flush<WN>(C.cb >= 0, C.cb, bv, row, nx);
-    C.reset();
+        for (int w = 0; w < WN; ++w) bv[w] = C.bs[w * kWave];
+        seg_flush<WN>(C.cb >= 0, C.cb, bv, row, nx);
+    }
 }
 
 // Two rows cached together: entries of 2*WN values, the first WN for row0's
@@ -513,11 +516,13 @@ __device__ __forceinline__ void cache_add_rows2(Cache2<2 * WN> &C, bool valid, i
         bool use_b = miss && !use_a;
         bool ev_a = use_a && C.ca >= 0;
         bool ev_b = use_b && C.cb >= 0;
-        int ecell = ev_a ? C.ca : C.cb;
-        double ev[W2];
+        if (__ballot(ev_a || ev_b)) {
+            int ecell = ev_a ? C.ca : C.cb;
+            double ev[W2];
 #pragma unroll
-        for (int w = 0; w < W2; ++w) ev[w] = ev_a ? C.a[w] : C.bs[w * kWave];
-        seg_flush_rows2<WN>(ev_a || ev_b, ecell, ev, row0, row1, nx);
+            for (int w = 0; w < W2; ++w) ev[w] = ev_a ? C.a[w] : C.bs[w * kWave];
+            seg_flush_rows2<WN>(ev_a || ev_b, ecell, ev, row0, row1, nx);
+        }
         if (use_a) {
             C.ca = cell;
 #pragma unroll
@@ -548,11 +553,12 @@ __device__ __forceinline__ void cache_drain_rows2(Cache2<2 * WN> &C, double *row
                                                   int nx)
 {
     seg_flush_rows2<WN>(C.ca >= 0, C.ca, C.a, row0, row1, nx);
-    double bv[2 * WN];
+    if (__ballot(C.cb >= 0)) {
+        double bv[2 * WN];
 #pragma unroll
-    for (int w = 0; w < 2 * WN; ++w) bv[w] = C.bs[w * kWave];
-    seg_flush_rows2<WN>(C.cb >= 0, C.cb, bv, row0, row1, nx);
-    C.reset();
+        for (int w = 0; w < 2 * WN; ++w) bv[w] = C.bs[w * kWave];
+        seg_flush_rows2<WN>(C.cb >= 0, C.cb, bv, row0, row1, nx);
+    }
 }
 
 }  // namespace gk

@@ -411,6 +411,25 @@ def test_gpu_save_and_resume(tmp_path):
         assert np.max(np.abs(got - ref)) <= 1e-11 * max(np.max(np.abs(ref)), 1.0)
 
 
+@pytest.mark.parametrize("nx", [2, 4, 6])
+@pytest.mark.parametrize("n", [1, 65, 3001])
+def test_gpu_deposits_on_the_smallest_grids(nx, n):
+    """Splines as wide as the grid or wider: a wave's sums wrap at the low side,
+    on two cells twice. Waves of one cell and of all of them, entries that are
+    never used and that are flushed."""
+    print(f"smallest grids: nx={nx}, n={n}", flush=True)
+    w = workloads.weibel_1d2v(n, seed=nx, nx=nx, sigma1=0.6, sigma2=0.4, degree=3)
+    w["b0"] = 0.3 + 0.1 * np.arange(nx)
+    h, pg, osp, o_parts, (o_e1, o_e2, o_b) = _setup_pair(w)
+    for name in ("operatorHp2", "operatorHp1", "operatorHp2"):
+        getattr(G, name)(h, 0.3)
+        getattr(osp, name)(0.3)
+        assert_rows_close(pg.array, o_parts, REL)
+        for c in (1, 2):
+            ref = osp.j(c)
+            assert np.max(np.abs(h.j_dofs[c - 1] - ref)) <= REL * max(np.max(np.abs(ref)), 1.0)
+
+
 @pytest.mark.parametrize("n", [131071, 131072, 131073, 700001])
 def test_gpu_particles_come_back_whole(n):
     """Downloads around the size from which several threads copy chunks (4 MiB:
