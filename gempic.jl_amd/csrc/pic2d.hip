@@ -34,13 +34,10 @@ namespace {
 constexpr int kGrid2Max = 4096;            // nx*ny of the device deposit (LDS grid)
 
 // launch shape of the evaluation kernels: threads per workgroup (the waves
-// of a workgroup share its staged field), workgroups per CU, and the largest
+// of a workgroup share its staged field), and the largest
 // field (doubles, both fields of evaluate_multiple together) staged in LDS
 #ifndef GEMPIC_EVAL_THREADS
 #define GEMPIC_EVAL_THREADS 1024
-#endif
-#ifndef GEMPIC_EVAL_BLOCKS_PER_CU
-#define GEMPIC_EVAL_BLOCKS_PER_CU 4
 #endif
 #ifndef GEMPIC_EVAL_STAGE_MAX
 #define GEMPIC_EVAL_STAGE_MAX 8192
@@ -255,6 +252,10 @@ __global__ void __launch_bounds__(1024) k_pmc2d_deposit(Pmc2Args a)
     }
 }
 
+// k / w, given rw = 1 / w: (k + 1/2) / w is at least 1 / (2 w) from an integer, for
+// the k below 9000 of a grid in LDS 200 times the rounding error
+__device__ __forceinline__ int row_of(int k, float rw) { return (int)(((float)k + 0.5f) * rw); }
+
 constexpr int kFlushPatches = 4, kFlushShared = 8;
 
 // Row stride of a deposit grid with halo (nx + P columns), congruent to 4
@@ -282,9 +283,11 @@ __host__ __device__ __forceinline__ int halo_stride(int nx, int p)
 // no order and sorted by cell: 242 and 129 with every deposit through the
 // cache and 4 waves a workgroup, 200 and 125 (8 waves; 4: 205 and 131;
 // without the quads 213 and 111); 300,000 at degree 2: 23.1 and 27.9, 19.5
-// and 21.2. The bytes' time at a copy's rate is 83.
+// and 21.2. The bytes' time at a copy's rate is 83. Degree 1 is held to 64 registers
+// (8 waves a SIMD): without that its schedule kept fewer loads in flight, 16,777,216
+// sorted particles on 32 x 32 92 us, with it 86.
 template <int P, bool PP>
-__global__ void __launch_bounds__(kWave *GEMPIC_DEP_WAVES_FAST) k_pmc2d_deposit_fast(Pmc2Args a)
+__global__ void __launch_bounds__(kWave *GEMPIC_DEP_WAVES_FAST, P == 1 ? 8 : 1) k_pmc2d_deposit_fast(Pmc2Args a)
 {
     constexpr int W = P + 1, WW = W * W;
     extern __shared__ double smem[];
@@ -416,17 +419,23 @@ __global__ void __launch_bounds__(kWave *GEMPIC_DEP_WAVES_FAST) k_pmc2d_deposit_
     }
     if (errs) atomicOr(a.err, errs);
     __syncthreads();
+    // the halo's columns, then its rows onto the grid's own
+    for (int k = threadIdx.x; k < P * (a.ny + P); k += blockDim.x) {
+        const int gy = k / P, gx = k - gy * P;
+        grid[gx + gy * S] += grid[a.nx + gx + gy * S];
+    }
+    __syncthreads();
+    const float rw = 1.0f / (float)a.nx;
+    for (int k = threadIdx.x; k < P * a.nx; k += blockDim.x) {
+        const int gy = row_of(k, rw), gx = k - gy * a.nx;
+        grid[gx + gy * S] += grid[gx + (a.ny + gy) * S];
+    }
+    __syncthreads();
     double *out = a.part + (size_t)blockIdx.x * a.nx * a.ny;
+#pragma unroll 4
     for (int k = threadIdx.x; k < a.nx * a.ny; k += blockDim.x) {
-        const int gy = k / a.nx, gx = k - gy * a.nx;
-        const double *g = grid + gx + gy * S;
-        double t = g[0];
-        if (gx < P) t += g[a.nx];
-        if (gy < P) {
-            t += g[a.ny * S];
-            if (gx < P) t += g[a.ny * S + a.nx];
-        }
-        out[k] = t;
+        const int gy = row_of(k, rw), gx = k - gy * a.nx;
+        out[k] = grid[gx + gy * S];
     }
 }
 
@@ -482,8 +491,10 @@ __global__ void __launch_bounds__(1024) k_pmc2d_eval(Pmc2Args a)
     const int sw = STAGE ? a.nx + P : a.nx;                 // row stride of the staged field
     if constexpr (STAGE) {
         const int ns = sw * (a.ny + P);
+        const float rw = 1.0f / (float)sw;
+#pragma unroll 4
         for (int k = threadIdx.x; k < ns; k += blockDim.x) {
-            const int gy = k / sw, gx = k - gy * sw;
+            const int gy = row_of(k, rw), gx = k - gy * sw;
             const int g = (gx < a.nx ? gx : gx - a.nx) + (gy < a.ny ? gy : gy - a.ny) * a.nx;
             if constexpr (MULTI) {
                 sfield[2 * k] = a.f1[g];
@@ -1865,9 +1876,17 @@ int pmc2_enqueue(int op, int degree, bool deterministic, Pmc2Args a, double *rho
             if (e != hipSuccess)
                 return abi_fail(GEMPIC_ERR_DEVICE, (std::string("2D evaluation: ") + hipGetErrorString(e)).c_str());
         }
+        // As many workgroups as are on the chip at once (two a CU, one where the
+        // registers leave no more: degree 3 with two fields), each staging the field
+        // for all its particles; more, which even out the ends, from 8 particles a
+        // thread on. us for evaluate_multiple on 64 x 64, degree 3, at 1, 2 and 4 a
+        // CU: 500,000 particles 9.9, 10.9, 11.4; 1,000,000 14.6, 15.4, 18.5; 4,000,000
+        // -, 41.2, 43.8; 16,777,216 -, 164, 156; degree 1 at 2 and 4: 1,000,000 11.1, 13.0;
+        // 4,000,000 23.1, 24.5; 16,777,216 108, 104.
         const int nt = GEMPIC_EVAL_THREADS;
-        const unsigned gb = (unsigned)std::max<int64_t>(
-            1, std::min<int64_t>((int64_t)cus * GEMPIC_EVAL_BLOCKS_PER_CU, (a.n + nt - 1) / nt));
+        int64_t most = (int64_t)cus * (multi && stage && degree == 3 ? 1 : 2);
+        while (most < (int64_t)cus * 4 && a.n > most * nt * 8) most *= 2;
+        const unsigned gb = (unsigned)std::max<int64_t>(1, std::min<int64_t>(most, (a.n + nt - 1) / nt));
 #define EV(P, M, S) hipLaunchKernelGGL((k_pmc2d_eval<P, M, S>), dim3(gb), dim3(nt), sh, s, a)
 #define EVD(M, S) do { if (degree == 1) EV(1, M, S); else if (degree == 2) EV(2, M, S); else EV(3, M, S); } while (0)
         if (multi) { if (stage) EVD(true, true); else EVD(true, false); }
