@@ -398,11 +398,12 @@ def test_gpu_pmc2d_device_forms(degree):
 
 
 @pytest.mark.parametrize("degree, nx, ny, n", [(3, 256, 16, 300001), (3, 4, 256, 65), (2, 3, 3, 1000003),
-                                               (1, 64, 64, 1000003), (3, 64, 64, 1)])
+                                               (1, 64, 64, 1000003), (3, 64, 64, 1), (3, 18, 227, 300001),
+                                               (1, 36, 113, 65537)])
 def test_gpu_pmc2d_deposit_in_mixed_orders(degree, nx, ny, n):
     """The fast deposit changes between its two ways inside a wave's particles:
-    runs of one cell, of few cells and of no order, on the widest, the highest
-    and the smallest grids; evaluate_multiple's halo on the same grids."""
+    runs of one cell, of few cells and of no order, on the widest, the highest,
+    the smallest and the largest grids; evaluate_multiple's halo on the same grids."""
     print(f"deposit orders: degree {degree}, {nx} x {ny}, n={n}", flush=True)
     rng = np.random.default_rng(nx + ny)
     bounds = (0.0, 3.0, -1.0, 1.0)
