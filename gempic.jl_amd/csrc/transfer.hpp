@@ -27,8 +27,9 @@ namespace gl {
 
 // One pool for the process: kThreads x 2 buffers of kChunk bytes, made by the
 // first large copy and given back with the last handle (acquire/release
-// count them). A copy holds the pool's lock, so copies of several threads
-// follow one another, as they would on the link.
+// count them). A copy whose stream is done holds the pool's lock, so copies of
+// several threads follow one another, as they would on the link; work that is
+// still to come, and making or giving up a handle beside others, wait for no copy.
 class TransferPool {
 public:
     static constexpr size_t kChunk = (size_t)2 << 20;
@@ -43,15 +44,12 @@ public:
         return *p;
     }
 
-    void acquire()
-    {
-        std::lock_guard<std::mutex> g(m_);
-        ++users_;
-    }
+    void acquire() { ++users_; }
     void release()
     {
+        if (--users_ > 0) return;
         std::lock_guard<std::mutex> g(m_);
-        if (--users_ == 0) free_all();
+        if (users_ == 0) free_all();           // (no other came meanwhile)
     }
 
     // dst <- src (device memory of `device`, ready once `after` is done);
@@ -62,9 +60,9 @@ public:
             const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, after);
             return e != hipSuccess ? e : hipStreamSynchronize(after);
         }
-        std::lock_guard<std::mutex> g(m_);
         hipError_t e = hipStreamSynchronize(after);
         if (e != hipSuccess) return e;
+        std::lock_guard<std::mutex> g(m_);
         if (!make(device)) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
         const size_t chunks = (bytes + kChunk - 1) / kChunk;
         std::atomic<size_t> next{0};
@@ -150,7 +148,8 @@ private:
     }
 
     std::mutex m_;
-    int users_ = 0, device_ = -1;
+    std::atomic<int> users_{0};
+    int device_ = -1;
     bool made_ = false;
     Lane lanes_[kThreads];
 };
