@@ -53,7 +53,7 @@ public:
     }
 
     // dst <- src (device memory of `device`, ready once `after` is done);
-    // returns when dst is written
+    // returns when dst is written; the calling thread's device stays as it is
     hipError_t to_host(void *dst, const void *src, size_t bytes, hipStream_t after, int device)
     {
         if (bytes < kLeast) {
@@ -63,6 +63,7 @@ public:
         hipError_t e = hipStreamSynchronize(after);
         if (e != hipSuccess) return e;
         std::lock_guard<std::mutex> g(m_);
+        OnDevice here(device);
         if (!make(device)) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
         const size_t chunks = (bytes + kChunk - 1) / kChunk;
         std::atomic<size_t> next{0};
@@ -107,6 +108,19 @@ public:
     }
 
 private:
+    struct OnDevice {
+        int was = -1, now;
+        explicit OnDevice(int d) : now(d)
+        {
+            if (hipGetDevice(&was) != hipSuccess) was = d;
+            if (was != d) (void)hipSetDevice(d);
+        }
+        ~OnDevice()
+        {
+            if (was != now) (void)hipSetDevice(was);
+        }
+    };
+
     struct Lane {
         hipStream_t stream = nullptr;
         hipEvent_t done[2] = {nullptr, nullptr};

@@ -1,6 +1,6 @@
 """The pool that copies large GPU arrays to the caller (csrc/transfer.hpp), built
 for the CPU against a stand-in for the HIP calls it makes: who waits for whom,
-what is copied and what is given back."""
+which device is current, what is copied and what is given back."""
 import os
 import shutil
 import subprocess
@@ -90,6 +90,13 @@ int main()
         CHECK(p.to_host(b.data(), a.data(), n, &s, 0) == hipSuccess);
         CHECK(a == b);
     }
+    // of another device than the calling thread's: its streams, and the thread's device stays
+    {
+        std::vector<unsigned char> a(3 * k, 7), b(3 * k);
+        FakeStream s{1, false};
+        CHECK(p.to_host(b.data(), a.data(), a.size(), &s, 1) == hipSuccess);
+        CHECK(a == b && device_now == 0 && wrong_device == 0);
+    }
     // while one thread waits for a stream that is not done: others make and give
     // up users, and copy
     std::vector<unsigned char> a(4 * k, 5), b(4 * k), c(4 * k);
@@ -118,7 +125,7 @@ int main()
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
-def test_transfer_pool_waits(tmp_path):
+def test_transfer_pool_waits_and_devices(tmp_path):
     (tmp_path / "hip").mkdir()
     (tmp_path / "hip" / "hip_runtime.h").write_text(HIP)
     (tmp_path / "main.cpp").write_text(MAIN)
