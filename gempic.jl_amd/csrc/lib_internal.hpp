@@ -17,7 +17,7 @@ constexpr int kPrefetch = GEMPIC_PASS_PREFETCH;
 static_assert(kPrefetch == 1 || kPrefetch == 2, "prefetch depth 1 or 2");
 constexpr int kNxMax = 256;               // largest 1D grid handled by the device path
 constexpr int kGroup = 16;                // workgroups per first-level reduction group
-constexpr int kEpiGroupsMax = 64;         // workgroups of the deposit-sum kernel
+constexpr int kEpiGroupsMax = 64;         // groups of a pass's partial rows at most
 constexpr int kAdjNxMax = 128;            // largest 1D grid of the reverse-mode kernels
 
 // grid slots (nx doubles each) of a splitting's device field buffer

@@ -535,6 +535,7 @@ __device__ __forceinline__ void pass1d_body(const PassArgs &a, int bid, double *
     constexpr int NQ = (P1 + 2) / 2;
     constexpr int W0 = P0 + 1, W1 = P1 + 1;
     static_assert(P0 <= kPad && P1 <= kPad, "LDS field padding must cover the spline support");
+    static_assert(!RUN || DEPMASK != 0u || !HE || HE_PREV || V1, "HE alone updates B in block 0: bid is not it in a run");
 
     const int nx = a.nx;
     const int tid = threadIdx.x;
@@ -954,8 +955,9 @@ __global__ void __launch_bounds__(kBlock, GEMPIC_PASS_MIN_WAVES) k_pass1d_batch(
 // particles 15.2, 14.3; 300,001 25.7, 23.3; 1,048,576 31.7, 29.6; 4,194,304
 // 61.7, 59.1.
 //
-// The batched passes of an ensemble keep it in two launches (k_epi1d_batch):
-// there a workgroup's wait for its count would hold its place from the next.
+// The batched passes of an ensemble keep it in two launches (k_epi1d_batch_sum
+// and k_epi1d_batch_fin): there a workgroup's wait for its count would hold its
+// place from the next.
 // ---------------------------------------------------------------------------
 
 // index r*nx + k of live entry e (the e-th entry of the rows in mask)
@@ -1391,7 +1393,9 @@ size_t pass_shmem_bytes(int nx, int mode)
     size_t tail = (size_t)NTAB * nx;
     if (tail < (size_t)kBlock) tail = kBlock;
     const size_t diag = (size_t)nx * 8 + 8 + tail;
-    return sizeof(double) * (pass > diag ? pass : diag);
+    const size_t b = sizeof(double) * (pass > diag ? pass : diag);
+    // a deposit pass ends with the field part in the same LDS
+    return dep ? std::max(b, epi_shmem_bytes(nx)) : b;
 }
 
 // ---------------------------------------------------------------------------
