@@ -989,9 +989,10 @@ F2Args f2_args(gempic_splitting2d *h, double dt)
 // against 710), 700 at 16,777,216: the ways meet at 14 % (measured; 11.5 % by
 // this rule), 1.2 % (1.0 %) and 0.6 % (0.7 %) listed.
 constexpr double f2_listed_most(int64_t n) { return 16384.0 + (double)n / 160.0; }
-// Steps between two predictions of it: with strips as often as the particles
-// are binned, since what they drift in that time counts.
-constexpr int kPredictEvery = 50;
+// Steps between two predictions of it: one takes 10 us of the stream (event
+// and gap included), 50 small steps 2000 to 4000, 10 of the large ones 4500 and
+// up. The more particles, the more a late change of path costs.
+constexpr int64_t f2_predict_every(int64_t n) { return n >= (int64_t)1 << 22 ? 10 : 50; }
 
 int f2_predict(gempic_splitting2d *h, double dt)
 {
@@ -1037,7 +1038,7 @@ int f2_choose(gempic_splitting2d *h, double dt, bool wait, bool &slow)
     if (!c.known || dt != c.dt) {
         rc = f2_predict(h, dt);
         if (!rc) rc = f2_take(h);
-    } else if (c.age >= (h->f2_strips > 1 ? kBinEvery : kPredictEvery)) {
+    } else if (c.age >= f2_predict_every(h->n)) {
         if (c.pending) {
             if (wait || hipEventQuery(c.done) == hipSuccess) rc = f2_take(h);
             else (void)hipGetLastError();           // "not ready" is no error

@@ -227,15 +227,15 @@ def test_gpu_2d3v_hot_particles_take_the_operators_passes(n, steps, fused):
         h.to_device()
 
 
-@pytest.mark.parametrize("nx, ny, turn, calls", [(64, 64, 0.05, (80,)), (64, 64, 0.05, (1,) * 25 + (55,)),
-                                                (48, 36, 0.0125, (300,))])
-def test_gpu_2d3v_path_changes_within_a_call(nx, ny, turn, calls):
-    """A beam that a uniform B3 turns from x2 to x1 and on (`turn` a step): along
+@pytest.mark.parametrize("nx, ny, calls", [(64, 64, (300,)), (64, 64, (1,) * 120 + (180,)), (48, 36, (300,))])
+def test_gpu_2d3v_path_changes_within_a_call(nx, ny, calls):
+    """A beam that a uniform B3 turns from x2 to x1 and on (0.0125 a step): along
     x1 it crosses 2.2 cells a step, along x2 a quarter. The step goes from one
-    pass to the operators' passes and back within a call (strips: looked at every
-    10 steps; whole grids in LDS: every 50), and the state and the currents stay
-    the oracle's. The charge is small, so rounding differences (3e-14 a step)
+    pass to the operators' passes and back within a call (looked at every 50
+    steps), on strips and with whole grids in LDS, and the state and the currents
+    stay the oracle's. The charge is small, so rounding differences (3e-14 a step)
     only add up."""
+    turn = 0.0125
     print(f"2d3v path changes: {nx} x {ny}, calls {calls}", flush=True)
     n, dt = 20001, 0.05
     w = _hot(n=n, nx=nx, ny=ny, L1=0.25 * nx, L2=2.0 * ny, seed=10, vscale=0.2, fscale=1e-3)
