@@ -104,7 +104,10 @@ struct Launch {
 //   24 instances of 65,536 to 524,288 particles in one ensemble, whose
 //   workgroups fill the chip together: 164, 175, 176, 181
 // An ensemble's instances keep their stand-alone partition (equal results);
-// its pass takes several such blocks per workgroup (k_pass1d_batch).
+// its pass takes several such blocks per workgroup (k_pass1d_batch), and a
+// block's start and drain were cut since: these 24 instances 159 now. Instances of
+// 131,072 to 262,144 particles still pay for it (24 of 262,144: 162, with (8, 0) and
+// the drain as it was 155); gempic_ensemble_autotune finds them a partition.
 constexpr int kPerThread = 4;
 constexpr int kFewBlocks = 512;
 

@@ -918,7 +918,8 @@ __global__ void __launch_bounds__(kBlock, GEMPIC_PASS_MIN_WAVES) k_pass1d(PassAr
 // workgroup takes several in turn, with the fields staged once and the next
 // block's first particles loaded before the drain. One block per workgroup, and
 // this (us a step): 24 instances of 65,536 to 524,288 particles 183, 172; 64 of
-// up to 1,048,576 746, 645, in the reference's arithmetic 825, 770.
+// up to 1,048,576 746, 645, in the reference's arithmetic 825, 770 (159, 600 and 713
+// since a block's drain was cut, cache_drain).
 template <int P0, int P1, int MODE>
 __global__ void __launch_bounds__(kBlock, GEMPIC_PASS_MIN_WAVES) k_pass1d_batch(BatchArgs b)
 {

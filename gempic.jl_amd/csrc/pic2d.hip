@@ -476,8 +476,8 @@ __global__ void k_pmc2d_reduce2(const double *part2, int splits, int nn, double 
 // read per node). The next particle's position is loaded while the current
 // one is evaluated; loading two or four ahead ran slower (16,777,216
 // particles: 186 and 256 us against 172). evaluate_multiple took 184 us with
-// its fields staged without a halo; bound by VALU issue (the reference's
-// rounding: no fused multiply-adds), at 3.1 TB/s.
+// its fields staged without a halo; bound by VALU issue (90 % of the cycles: the
+// reference's rounding, no fused multiply-adds; LDS 74 %), at 3.4 TB/s.
 template <int P, bool MULTI, bool STAGE>
 __global__ void __launch_bounds__(1024) k_pmc2d_eval(Pmc2Args a)
 {

@@ -20,9 +20,11 @@
 // cell in a push, are put on a list and done from global memory by a kernel of
 // its own (in the pass itself, the general form's registers made it spill).
 //
-// Bound by LDS: per particle 148 reads (7 lanes per cycle and CU at random
-// nodes) and 68 to 80 atomic adds (3.5 per cycle; measured alone), which the
-// shared row sums below keep down: B1's rows serve Hp3 and the neighbouring
+// Bound by LDS: at degree 3, 127 reads per particle and 7 more for each of the
+// three pushes that crosses a cell, 68 to 80 atomic adds; its pipe is busy 97 % of
+// a CU's cycles, 50 per particle, 46 % of the cycles in bank conflicts of lanes at
+// random nodes (VALU 26 %; counters at 16,777,216 particles, 64 x 64). The shared row sums below
+// keep the reads down: B1's rows serve Hp3 and the neighbouring
 // Hp2, and a path that stays in its cell deposits 3 rows, not 4.
 #pragma once
 

@@ -509,8 +509,8 @@ int gempic_maxwell2d_compute_e_from_rho(gempic_maxwell2d *m, const double *rho, 
  *   operatorHE: v += dt qm E(x), then compute_b_from_e! (:423-444);
  *   operatorHB: compute_e_from_b! (:370-412);
  *   strang_splitting: HB HE Hp3 Hp2 Hp1 Hp2 Hp3 HE HB (half steps around Hp1).
- * Particles are kept sorted by cell on the device (every `interval` steps,
- * default 20); get_particles restores the caller's order. Degrees 1..3,
+ * The device keeps the particles in an order of its own (below);
+ * get_particles restores the caller's order. Degrees 1..3,
  * 2*degree+1 <= nx, ny and nx*ny <= 4096. The current deposits add in an
  * order that depends on timing between wave flushes: results agree with the
  * oracle to rounding, not bitwise.
@@ -544,7 +544,11 @@ int gempic_splitting2d_strang_splitting(gempic_splitting2d *h, double dt, int64_
 int gempic_splitting2d_step_counts(gempic_splitting2d *h, int64_t *fused, int64_t *operators);
 int gempic_splitting2d_synchronize(gempic_splitting2d *h);
 /* sort the particles by cell every `interval` Strang steps (0, the default:
-   never; the passes run faster on unordered particles) */
+   never; the passes run faster on unordered particles). On grids whose nine
+   fields do not fit in a workgroup's LDS together (64 x 64 at degree 3), Strang
+   steps that run as one pass bin the particles by strips of rows every 10 steps,
+   in an order that varies from run to run; a sort is then undone by the next
+   binning and only costs. */
 int gempic_splitting2d_set_sort_interval(gempic_splitting2d *h, int64_t interval);
 /* add_charge! (particle_mesh_coupling_2d.jl:94-105) of the handle's particles
  * with degree (p, p) and q = charge w common_weight, into rho (nx*ny, not
