@@ -647,7 +647,7 @@ __global__ void __launch_bounds__(256) k_f2_rest(F2Args a, int nblocks, double *
 // cell; with strips, binned now, those that begin after it has left the rows
 // held. Groups of 64 neighbouring particles, every stride-th, stand for all: of
 // 262,144 particles, 1 % to be listed are found to 4 % of that. Latency: 5 to 8 us
-// (a million particles: 16), against the 600 to 16,000 of the steps up to the next.
+// (a million particles: 16), against the 2000 and more of the steps up to the next.
 constexpr int kPredictBlocks = 256;
 constexpr int64_t kPredictSample = (int64_t)1 << 18;
 
